@@ -533,7 +533,190 @@ __global__ void k_bvh_small(BuildDev B, uint32_t* idx, uint32_t nsmall) {
     }
 }
 
+// ---------------------------------------------------------------- wide tree
+// The children of the wide node that stands for binary node `open`: that
+// node's, and while there is room the interior child with the largest surface
+// area gives way to its own two children (large boxes are entered most often,
+// so opening them saves the most node visits).
+struct WideKids {
+    float box[4][6];
+    uint32_t ref[4], cnt[4];  // as in the binary node: count 0 for an interior child
+    int n;
+    uint32_t inner;  // interior children
+};
+__host__ __device__ inline float bits_float(uint32_t v) { return __builtin_bit_cast(float, v); }
+__host__ __device__ inline WideKids wide_open(const uint4* binary, uint32_t open) {
+    WideKids w;
+    int n = 0, at = 0;
+    while (true) {
+        const uint4* b = binary + (size_t)open * 4;
+        const uint4 q0 = b[0], q1 = b[1], q2 = b[2], q3 = b[3];
+        const uint32_t q[16] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+        bool first = true;  // the first child takes the opened child's place
+        for (int c = 0; c < 2; ++c) {
+            if (q[12 + c] == kEmptyRef) continue;
+            const int s = first ? at : n;
+            if (s == n) ++n;
+            first = false;
+            for (int k = 0; k < 6; ++k) w.box[s][k] = bits_float(q[6 * c + k]);
+            w.ref[s] = q[12 + c];
+            w.cnt[s] = q[14 + c];
+        }
+        at = -1;
+        float big = -1.f;
+        for (int s = 0; s < n && n < 4; ++s) {
+            const float x = w.box[s][3] - w.box[s][0], y = w.box[s][4] - w.box[s][1], z = w.box[s][5] - w.box[s][2];
+            const float area = x * y + y * z + z * x;
+            if (w.cnt[s] == 0 && !(area <= big)) {
+                big = area;
+                at = s;
+            }
+        }
+        if (at < 0) break;
+        open = w.ref[at];
+    }
+    w.n = n;
+    w.inner = 0;
+    for (int s = 0; s < n; ++s) w.inner += w.cnt[s] == 0 ? 1u : 0u;
+    return w;
+}
+// The node with those children, the interior ones at `next` and on.
+__host__ __device__ inline gyd::WideNode wide_make(const WideKids& w, uint32_t next) {
+    // the children's grid: 255 steps an axis, the node's box between steps 2
+    // and 252 (FP32 places the origin within two steps, since a padded box is
+    // at least 60 ulp wide); bytes are rounded outward with 1/128 step to spare
+    // for the traversal's FP32 distances
+    gyd::WideNode o;
+    for (int k = 0; k < 6; ++k) o.q[k] = 0u;
+    for (int k = 0; k < 3; ++k) {
+        float lo = __builtin_huge_valf(), hi = -__builtin_huge_valf();
+        for (int s = 0; s < w.n; ++s) {
+            lo = fminf(lo, w.box[s][k]);
+            hi = fmaxf(hi, w.box[s][3 + k]);
+        }
+        const float step = fmaxf((hi - lo) * (1.f / 250.f), 1e-30f);
+        o.org[k] = lo - 2.f * step;
+        o.scale[k] = step * 16777216.f;
+        for (int s = 0; s < 4; ++s) {
+            int mn = 255, mx = 0;  // absent: inverted
+            if (s < w.n) {
+                mn = (int)floor(((double)w.box[s][k] - (double)o.org[k]) / (double)step - 0.0078125);
+                mx = (int)ceil(((double)w.box[s][3 + k] - (double)o.org[k]) / (double)step + 0.0078125);
+                mn = mn < 0 ? 0 : (mn > 255 ? 255 : mn);
+                mx = mx < 0 ? 0 : (mx > 255 ? 255 : mx);
+            }
+            o.q[2 * k] |= (uint32_t)mn << (8 * s);
+            o.q[2 * k + 1] |= (uint32_t)mx << (8 * s);
+        }
+    }
+    for (int s = 0; s < 4; ++s) {
+        if (s >= w.n) o.entry[s] = gyd::kTravLeaf;  // an empty leaf
+        else if (w.cnt[s] == 0) o.entry[s] = next++;
+        else o.entry[s] = gyd::kTravLeaf | (w.cnt[s] << 27) | w.ref[s];
+    }
+    return o;
+}
+
+// One level of the wide tree: node w of the level stands for the binary node
+// src[w].  ctr: nodes so far, level begin, level end, levels.  The order of the
+// nodes of a level is not fixed; no result depends on it.  1.31M triangles:
+// 0.44M nodes from 1.31M.
+__global__ void __launch_bounds__(64) k_wide_level(const uint4* __restrict__ binary, gyd::WideNode* __restrict__ wide,
+                                                   uint32_t* __restrict__ src, uint32_t* __restrict__ ctr) {
+    const uint32_t end = ctr[2];
+    for (uint32_t w = ctr[1] + blockIdx.x * 64 + threadIdx.x; w < end; w += gridDim.x * 64) {
+        const WideKids kids = wide_open(binary, src[w]);
+        const uint32_t next = kids.inner ? atomicAdd(&ctr[0], kids.inner) : 0u;
+        wide[w] = wide_make(kids, next);
+        uint32_t i = next;
+        for (int s = 0; s < kids.n; ++s)
+            if (kids.cnt[s] == 0) src[i++] = kids.ref[s];
+    }
+}
+__global__ void k_wide_advance(uint32_t* ctr) {
+    if (threadIdx.x != 0) return;
+    if (ctr[2] > ctr[1]) ++ctr[3];
+    ctr[1] = ctr[2];
+    ctr[2] = ctr[0];
+}
+__global__ void k_wide_root(uint32_t* src, uint32_t* ctr) {
+    if (threadIdx.x != 0) return;
+    src[0] = 0u;
+    ctr[0] = 1u;
+    ctr[1] = 0u;
+    ctr[2] = 1u;
+    ctr[3] = 0u;
+}
+
 }  // namespace
+
+// Small trees are collapsed on the host: up to kWideHost nodes (a few tens of
+// microseconds) the device's launches, allocations and read-back (0.2 ms) would
+// cost more.
+constexpr int64_t kWideHost = 1024;
+static int BuildWideHost(Ctx* c, const std::vector<uint32_t>& nodes, void** wide, int64_t* n_wide, int* depth) {
+    std::vector<gyd::WideNode> out;
+    std::vector<uint32_t> src(1, 0u);
+    const uint4* binary = reinterpret_cast<const uint4*>(nodes.data());
+    size_t begin = 0;
+    *depth = 0;
+    while (begin < src.size()) {  // a level
+        const size_t end = src.size();
+        for (; begin < end; ++begin) {
+            const WideKids kids = wide_open(binary, src[begin]);
+            out.push_back(wide_make(kids, (uint32_t)src.size()));
+            for (int s = 0; s < kids.n; ++s)
+                if (kids.cnt[s] == 0) src.push_back(kids.ref[s]);
+        }
+        ++*depth;
+    }
+    *n_wide = (int64_t)out.size();
+    return Upload(c, wide, out.data(), out.size() * sizeof(gyd::WideNode));
+}
+
+int BuildWideBVH(Ctx* c, const std::vector<uint32_t>& nodes, int max_depth, void** wide, int64_t* n_wide, int* depth) {
+    const int64_t n_binary = (int64_t)(nodes.size() / 16);
+    if (n_binary <= kWideHost) return BuildWideHost(c, nodes, wide, n_wide, depth);
+    *wide = nullptr;
+    void *binary = nullptr, *tmp = nullptr, *src = nullptr, *ctr = nullptr;
+    int rc = Upload(c, &binary, nodes.data(), nodes.size() * 4);
+    // each wide node stands for a binary node of its own
+    if (rc == GY_OK) rc = DevAlloc(c, &tmp, (size_t)n_binary * sizeof(gyd::WideNode));
+    if (rc == GY_OK) rc = DevAlloc(c, &src, (size_t)n_binary * 4);
+    if (rc == GY_OK) rc = DevAlloc(c, &ctr, 16);
+    uint32_t h[4] = {0, 0, 0, 0};
+    if (rc == GY_OK) {
+        const unsigned blocks = (unsigned)std::min<int64_t>((n_binary + 63) / 64, 4096);
+        hipLaunchKernelGGL(k_wide_root, dim3(1), dim3(64), 0, c->stream, (uint32_t*)src, (uint32_t*)ctr);
+        for (int l = 0; l <= max_depth; ++l) {
+            hipLaunchKernelGGL(k_wide_level, dim3(blocks), dim3(64), 0, c->stream, (const uint4*)binary, (gyd::WideNode*)tmp, (uint32_t*)src, (uint32_t*)ctr);
+            hipLaunchKernelGGL(k_wide_advance, dim3(1), dim3(64), 0, c->stream, (uint32_t*)ctr);
+        }
+        rc = CheckLaunch(c, "wide bvh");
+        hipError_t e = hipMemcpyAsync(h, ctr, 16, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        if (rc == GY_OK && e != hipSuccess) rc = HipFail(e, "wide bvh");
+        if (rc == GY_OK && h[1] != h[2]) rc = Fail(GY_ERR_DEVICE, "wide bvh: levels left over");
+    }
+    if (rc == GY_OK) rc = DevAlloc(c, wide, (size_t)h[0] * sizeof(gyd::WideNode));
+    if (rc == GY_OK) {
+        hipError_t e = hipMemcpyAsync(*wide, tmp, (size_t)h[0] * sizeof(gyd::WideNode), hipMemcpyDeviceToDevice, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        if (e != hipSuccess) rc = HipFail(e, "wide bvh copy");
+    }
+    DevFree(binary);
+    DevFree(tmp);
+    DevFree(src);
+    DevFree(ctr);
+    if (rc != GY_OK) {
+        DevFree(*wide);
+        *wide = nullptr;
+        return rc;
+    }
+    *n_wide = h[0];
+    *depth = (int)h[3];
+    return GY_OK;
+}
 
 // Build on the device, then copy nodes and leaf order back for the scene upload.
 int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, BVHBuild* out) {

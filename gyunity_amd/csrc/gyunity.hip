@@ -143,14 +143,14 @@ void TimersCollect(Ctx* c) {
 template <int STACK, bool SPH>
 __global__ void __launch_bounds__(256) k_trace_closest(SceneDev S, const gy_ray* __restrict__ rays, int64_t n,
                                                        gy_hit* __restrict__ hits) {
-    __shared__ uint32_t stack[STACK * 256];
+    __shared__ uint32_t stack[kPathLds * 256];
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float4* rp = reinterpret_cast<const float4*>(rays + i);
     const float4 a = rp[0], b = rp[1];
     Hit h;
     gy_hit out;
-    if (traverse<false, STACK, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, blockDim.x)) {
+    if (find_hit<false, STACK, false, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256)) {
         out.t = h.t;
         out.prim = h.prim;
         out.b1 = h.b1;
@@ -167,13 +167,13 @@ __global__ void __launch_bounds__(256) k_trace_closest(SceneDev S, const gy_ray*
 template <int STACK, bool SPH>
 __global__ void __launch_bounds__(256) k_trace_any(SceneDev S, const gy_ray* __restrict__ rays, int64_t n,
                                                    int32_t* __restrict__ occ) {
-    __shared__ uint32_t stack[STACK * 256];
+    __shared__ uint32_t stack[kPathLds * 256];
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float4* rp = reinterpret_cast<const float4*>(rays + i);
     const float4 a = rp[0], b = rp[1];
     Hit h;
-    occ[i] = traverse<true, STACK, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, blockDim.x) ? 1 : 0;
+    occ[i] = find_hit<true, STACK, false, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256) ? 1 : 0;
 }
 
 __device__ inline void wave_add_u64(unsigned long long* dst, uint64_t v) {
@@ -185,14 +185,14 @@ __device__ inline void wave_add_u64(unsigned long long* dst, uint64_t v) {
 template <int STACK, bool SPH>
 __global__ void __launch_bounds__(256) k_count_visits(SceneDev S, const gy_ray* __restrict__ rays, int64_t n,
                                                       unsigned long long* counters) {
-    __shared__ uint32_t stack[STACK * 256];
+    __shared__ uint32_t stack[kPathLds * 256];
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t nn = 0, nt = 0;
     if (i < n) {
         const float4* rp = reinterpret_cast<const float4*>(rays + i);
         const float4 a = rp[0], b = rp[1];
         Hit h;
-        traverse<false, STACK, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, blockDim.x, &nn, &nt);
+        find_hit<false, STACK, true, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256, &nn, &nt);
     }
     wave_add_u64(&counters[0], nn);
     wave_add_u64(&counters[1], nt);
@@ -205,7 +205,7 @@ template <int STACK, int BLOCK, bool ENV, bool SPH>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
 k_pt_megakernel(SceneDev S, PathParams P, FilmDev F, int s0, int n_s,
                                                          unsigned long long* counters) {
-    __shared__ uint32_t stack[STACK * BLOCK];
+    __shared__ uint32_t stack[kPathLds * BLOCK];
     const int64_t t = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     int s_local, px, py;
     pass_pixel(F, t, &s_local, &px, &py);
@@ -224,7 +224,7 @@ k_pt_megakernel(SceneDev S, PathParams P, FilmDev F, int s0, int n_s,
 template <int STACK, int BLOCK, bool ENV, bool SPH>
 __global__ void __launch_bounds__(BLOCK) k_pt_count(SceneDev S, PathParams P, FilmDev F, int s0, int n_s,
                                                     unsigned long long* counters) {
-    __shared__ uint32_t stack[STACK * BLOCK];
+    __shared__ uint32_t stack[kPathLds * BLOCK];
     const int64_t t = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     int s_local, px, py;
     pass_pixel(F, t, &s_local, &px, &py);
@@ -247,7 +247,7 @@ template <int STACK, bool ENV, bool SPH>
 __global__ void __launch_bounds__(128) k_li_samples(SceneDev S, PathParams P, int n, const int32_t* __restrict__ xs,
                                                     const int32_t* __restrict__ ys, const int32_t* __restrict__ ss,
                                                     float* __restrict__ L, float* __restrict__ raster, int32_t* __restrict__ dims) {
-    __shared__ uint32_t stack[STACK * 128];
+    __shared__ uint32_t stack[kPathLds * 128];
     const int i = blockIdx.x * 128 + threadIdx.x;
     if (i >= n) return;
     PathCounters pc = {};
@@ -267,7 +267,7 @@ __global__ void __launch_bounds__(128) k_li_samples(SceneDev S, PathParams P, in
 template <int STACK, int BLOCK, bool ENV>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) k_lt(SceneDev S, PathParams P, LightCamDev C, int64_t n, float total,
                                               float* __restrict__ splat) {
-    __shared__ uint32_t stack[STACK * BLOCK];
+    __shared__ uint32_t stack[kPathLds * BLOCK];
     const int64_t t = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     if (t >= n) return;
     lt_path<STACK, ENV>(S, P, C, (uint64_t)t, total, splat, stack + threadIdx.x, BLOCK);
@@ -339,16 +339,16 @@ int LaunchTraceAnyT(Ctx* c, const SceneDev& S, const gy_ray* rays, int64_t n, in
 int LaunchTraceClosest(Ctx* c, Scene* sc, const gy_ray* rays, int64_t n, gy_hit* hits) {
     if (n <= 0) return GY_OK;
     if (sc->dev.n_sph > 0)
-        return sc->stack <= 32 ? LaunchTraceClosestT<32, true>(c, sc->dev, rays, n, hits)
-                               : LaunchTraceClosestT<64, true>(c, sc->dev, rays, n, hits);
-    return sc->stack <= 32 ? LaunchTraceClosestT<32, false>(c, sc->dev, rays, n, hits)
-                           : LaunchTraceClosestT<64, false>(c, sc->dev, rays, n, hits);
+        return sc->stack <= 64 ? LaunchTraceClosestT<64, true>(c, sc->dev, rays, n, hits)
+                               : LaunchTraceClosestT<192, true>(c, sc->dev, rays, n, hits);
+    return sc->stack <= 64 ? LaunchTraceClosestT<64, false>(c, sc->dev, rays, n, hits)
+                           : LaunchTraceClosestT<192, false>(c, sc->dev, rays, n, hits);
 }
 int LaunchTraceAny(Ctx* c, Scene* sc, const gy_ray* rays, int64_t n, int32_t* occ) {
     if (n <= 0) return GY_OK;
     if (sc->dev.n_sph > 0)
-        return sc->stack <= 32 ? LaunchTraceAnyT<32, true>(c, sc->dev, rays, n, occ) : LaunchTraceAnyT<64, true>(c, sc->dev, rays, n, occ);
-    return sc->stack <= 32 ? LaunchTraceAnyT<32, false>(c, sc->dev, rays, n, occ) : LaunchTraceAnyT<64, false>(c, sc->dev, rays, n, occ);
+        return sc->stack <= 64 ? LaunchTraceAnyT<64, true>(c, sc->dev, rays, n, occ) : LaunchTraceAnyT<192, true>(c, sc->dev, rays, n, occ);
+    return sc->stack <= 64 ? LaunchTraceAnyT<64, false>(c, sc->dev, rays, n, occ) : LaunchTraceAnyT<192, false>(c, sc->dev, rays, n, occ);
 }
 
 // ------------------------------------------------------------------ scene upload
@@ -529,7 +529,6 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
         delete sc;
         return Fail(GY_ERR_UNSUPPORTED, "BVH deeper than the 64-entry traversal stack");
     }
-    sc->stack = (b.max_depth + 1 <= 32) ? 32 : 64;
     // Pad every child box outward so that the traversal never rejects a box
     // containing a triangle the triangle test accepts (rounding in that test
     // can place an accepted hit slightly outside the triangle).
@@ -576,10 +575,16 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     if ((rc = Upload(c, &p, shade.data(), shade.size() * sizeof(float4))) != GY_OK) goto fail;
     sc->d_shade = p;
     sc->dev.shade = (const float4*)p;
-    if ((rc = Upload(c, &p, b.nodes.data(), b.nodes.size() * 4)) != GY_OK) goto fail;
-    sc->d_nodes = p;
-    sc->dev.nodes = (const uint4*)p;
-    sc->dev.n_nodes = (int32_t)(b.nodes.size() / 16);
+    {
+        int64_t n_wide = 0;
+        int depth = 0;
+        if ((rc = BuildWideBVH(c, b.nodes, b.max_depth, &p, &n_wide, &depth)) != GY_OK) goto fail;
+        sc->d_nodes = p;
+        sc->dev.nodes = (const WideNode*)p;
+        sc->dev.n_nodes = (int32_t)n_wide;
+        // the end mark, and at most three children of each node on a path
+        sc->stack = 1 + 3 * depth <= kStackSmall ? kStackSmall : kStackLarge;
+    }
     if ((rc = Upload(c, &p, d.mats, (size_t)d.n_mat * GY_MAT_WORDS * 4)) != GY_OK) goto fail;
     sc->d_mats = p;
     sc->dev.mats = (const uint32_t*)p;
@@ -789,15 +794,15 @@ int LaunchMegaT(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, i
 int LaunchMegaFilm(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, int s0, int n_s, int block, bool count,
                    bool timed) {
     if (sc->dev.n_sph > 0)
-        return sc->stack <= 32 ? LaunchMegaT<32, 128, true>(c, sc, film, P, s0, n_s, count, timed)
-                               : LaunchMegaT<64, 128, true>(c, sc, film, P, s0, n_s, count, timed);
-    if (sc->stack <= 32) {
-        if (block == 64) return LaunchMegaT<32, 64, false>(c, sc, film, P, s0, n_s, count, timed);
-        if (block == 256) return LaunchMegaT<32, 256, false>(c, sc, film, P, s0, n_s, count, timed);
-        return LaunchMegaT<32, 128, false>(c, sc, film, P, s0, n_s, count, timed);
+        return sc->stack <= 64 ? LaunchMegaT<64, 128, true>(c, sc, film, P, s0, n_s, count, timed)
+                               : LaunchMegaT<192, 128, true>(c, sc, film, P, s0, n_s, count, timed);
+    if (sc->stack <= 64) {
+        if (block == 64) return LaunchMegaT<64, 64, false>(c, sc, film, P, s0, n_s, count, timed);
+        if (block == 256) return LaunchMegaT<64, 256, false>(c, sc, film, P, s0, n_s, count, timed);
+        return LaunchMegaT<64, 128, false>(c, sc, film, P, s0, n_s, count, timed);
     }
-    if (block == 64) return LaunchMegaT<64, 64, false>(c, sc, film, P, s0, n_s, count, timed);
-    return LaunchMegaT<64, 128, false>(c, sc, film, P, s0, n_s, count, timed);
+    if (block == 64) return LaunchMegaT<192, 64, false>(c, sc, film, P, s0, n_s, count, timed);
+    return LaunchMegaT<192, 128, false>(c, sc, film, P, s0, n_s, count, timed);
 }
 
 int LaunchMega(Ctx* c, Scene* sc, const PathParams& P, int s0, int n_s, int block, bool count) {
@@ -1179,11 +1184,11 @@ extern "C" int gy_render_light_tracing(gy_scene* s, const gy_camera_desc* cam, c
         const unsigned blocks = (unsigned)((n + bs - 1) / bs);
         void (*kern)(SceneDev, PathParams, LightCamDev, int64_t, float, float*);
         if (sc->dev.env.w > 0)
-            kern = sc->stack <= 32 ? (bs == 64 ? k_lt<32, 64, true> : bs == 256 ? k_lt<32, 256, true> : k_lt<32, 128, true>)
-                                   : (bs == 64 ? k_lt<64, 64, true> : bs == 256 ? k_lt<64, 256, true> : k_lt<64, 128, true>);
+            kern = sc->stack <= 64 ? (bs == 64 ? k_lt<64, 64, true> : bs == 256 ? k_lt<64, 256, true> : k_lt<64, 128, true>)
+                                   : (bs == 64 ? k_lt<192, 64, true> : bs == 256 ? k_lt<192, 256, true> : k_lt<192, 128, true>);
         else
-            kern = sc->stack <= 32 ? (bs == 64 ? k_lt<32, 64, false> : bs == 256 ? k_lt<32, 256, false> : k_lt<32, 128, false>)
-                                   : (bs == 64 ? k_lt<64, 64, false> : bs == 256 ? k_lt<64, 256, false> : k_lt<64, 128, false>);
+            kern = sc->stack <= 64 ? (bs == 64 ? k_lt<64, 64, false> : bs == 256 ? k_lt<64, 256, false> : k_lt<64, 128, false>)
+                                   : (bs == 64 ? k_lt<192, 64, false> : bs == 256 ? k_lt<192, 256, false> : k_lt<192, 128, false>);
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(bs), 0, c->stream, sc->dev, P, C, n, (float)n, (float*)d);
         rc = CheckLaunch(c, "k_lt");
     }
@@ -1312,8 +1317,8 @@ extern "C" int gy_count_visits(gy_scene* s, const gy_ray* rays, int64_t n, int64
     if (rc != GY_OK) return rc;
     if (n > 0) {
         const bool sph = sc->dev.n_sph > 0;
-        auto kern = sc->stack <= 32 ? (sph ? k_count_visits<32, true> : k_count_visits<32, false>)
-                                    : (sph ? k_count_visits<64, true> : k_count_visits<64, false>);
+        auto kern = sc->stack <= 64 ? (sph ? k_count_visits<64, true> : k_count_visits<64, false>)
+                                    : (sph ? k_count_visits<192, true> : k_count_visits<192, false>);
         hipLaunchKernelGGL(kern, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, sc->dev,
                            (const gy_ray*)c->rays.ptr, n, (unsigned long long*)c->ctr.ptr);
         rc = CheckLaunch(c, "k_count_visits");
@@ -1559,11 +1564,11 @@ extern "C" int gy_li_samples(gy_scene* s, const gy_camera_desc* cam, const gy_re
     if (rc == GY_OK) {
         const unsigned blocks = (unsigned)((n + 127) / 128);
         const bool env = sc->dev.env.w > 0;
-        auto kern = sc->stack <= 32 ? (env ? k_li_samples<32, true, false> : k_li_samples<32, false, false>)
-                                    : (env ? k_li_samples<64, true, false> : k_li_samples<64, false, false>);
+        auto kern = sc->stack <= 64 ? (env ? k_li_samples<64, true, false> : k_li_samples<64, false, false>)
+                                    : (env ? k_li_samples<192, true, false> : k_li_samples<192, false, false>);
         if (sc->dev.n_sph > 0)
-            kern = sc->stack <= 32 ? (env ? k_li_samples<32, true, true> : k_li_samples<32, false, true>)
-                                   : (env ? k_li_samples<64, true, true> : k_li_samples<64, false, true>);
+            kern = sc->stack <= 64 ? (env ? k_li_samples<64, true, true> : k_li_samples<64, false, true>)
+                                   : (env ? k_li_samples<192, true, true> : k_li_samples<192, false, true>);
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(128), 0, c->stream, sc->dev, P, n, (const int32_t*)dx, (const int32_t*)dy,
                            (const int32_t*)ds, (float*)dL, (float*)dr, (int32_t*)dd);
         rc = CheckLaunch(c, "k_li_samples");

@@ -21,6 +21,10 @@ enum KernelCategory {
     kKernOther = 7
 };
 
+// Traversal stack capacities (entries per lane).  Binary trees are at most 63
+// levels deep, so the wide tree's three entries a level stay below kStackLarge.
+constexpr int kStackSmall = 64, kStackLarge = 192;
+
 struct DevBuf {
     void* ptr = nullptr;
     size_t bytes = 0;
@@ -89,7 +93,7 @@ struct Scene {
     float world_lo[3] = {0, 0, 0}, world_hi[3] = {0, 0, 0};
     std::vector<int32_t> area_tri;  // area lights as created (the environment light follows them)
     std::vector<float> area_le, area_func;
-    int stack = 64;
+    int stack = kStackLarge;  // entries the traversal stack of this tree can need: kStackSmall or kStackLarge
     gy_scene_stats stats = {};
     double upload_ms = 0.0;
     std::vector<uint32_t> host_nodes;
@@ -184,5 +188,8 @@ int BatchAdjoint(Ctx* c, Batch* b, const float* dimages, float* grad_tex, float*
 int BatchImages(Ctx* c, Batch* b, float* images);
 // GPU binned-SAH BVH build (bvh_gpu.hip).
 int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, BVHBuild* out);
+// The traversal tree of a binary tree (bvh_gpu.hip): n_wide WideNode records on
+// the device in *wide, `depth` levels.
+int BuildWideBVH(Ctx* c, const std::vector<uint32_t>& nodes, int max_depth, void** wide, int64_t* n_wide, int* depth);
 
 }  // namespace gy

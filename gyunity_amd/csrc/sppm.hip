@@ -123,7 +123,7 @@ __device__ inline uint32_t ordered(float f) {  // float -> uint32 with the same 
 // faster per iteration on the reference's settings.
 template <int STACK>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4))) k_sppm_eye(gyd::SceneDev S, PathParams P, SppmDev D, int iter) {
-    __shared__ uint32_t stack[STACK * 128];
+    __shared__ uint32_t stack[kPathLds * 128];
     const int64_t p = (int64_t)blockIdx.x * 128 + threadIdx.x;
     if (p >= (int64_t)D.W * D.H) return;
     const int px = (int)(p % D.W), py = (int)(p / D.W);
@@ -258,7 +258,7 @@ __global__ void k_sppm_grid(SppmDev D, GridDev G, uint32_t* counts) {
 template <int STACK>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5))) k_sppm_trace(gyd::SceneDev S, PathParams P, VtxDev V, int iter0, int n_iter,
                                                     int64_t photons) {
-    __shared__ uint32_t stack[STACK * 128];
+    __shared__ uint32_t stack[kPathLds * 128];
     const int64_t t = (int64_t)blockIdx.x * 128 + threadIdx.x;
     if ((int64_t)blockIdx.x * 128 >= photons * n_iter) return;  // workgroup-uniform
     const bool valid = t < photons * n_iter;
@@ -590,7 +590,7 @@ extern "C" int gy_render_sppm(gy_scene* s, const gy_camera_desc* cam, const gy_s
     };
     int end_bit = 32;
     while ((1ll << (end_bit - 32)) < WH) ++end_bit;
-    const bool stack64 = sc->stack > 32;
+    const bool stack64 = sc->stack > 64;
     // Photon vertices: one list per iteration of a chunk of iterations traced
     // together (photons_per_launch photon paths per launch, about 4M by
     // default), grown and traced again when a list overflows; the chunk
@@ -631,10 +631,10 @@ extern "C" int gy_render_sppm(gy_scene* s, const gy_camera_desc* cam, const gy_s
                 n_iter = std::min(chunk, sp->iterations - iter0);
                 hipLaunchKernelGGL(k_u32_fill, dim3(1), dim3(256), 0, c->stream, vcount, 0u, (int64_t)n_iter);
                 if (stack64)
-                    hipLaunchKernelGGL(k_sppm_trace<64>, dim3(G1(photons * n_iter, 128)), dim3(128), 0, c->stream, sc->dev, P,
+                    hipLaunchKernelGGL(k_sppm_trace<192>, dim3(G1(photons * n_iter, 128)), dim3(128), 0, c->stream, sc->dev, P,
                                        VtxDev{vtx, vcount, vcap}, iter0, n_iter, photons);
                 else
-                    hipLaunchKernelGGL(k_sppm_trace<32>, dim3(G1(photons * n_iter, 128)), dim3(128), 0, c->stream, sc->dev, P,
+                    hipLaunchKernelGGL(k_sppm_trace<64>, dim3(G1(photons * n_iter, 128)), dim3(128), 0, c->stream, sc->dev, P,
                                        VtxDev{vtx, vcount, vcap}, iter0, n_iter, photons);
                 rc = CheckLaunch(c, "k_sppm_trace");
                 if (rc != GY_OK) break;
@@ -653,8 +653,8 @@ extern "C" int gy_render_sppm(gy_scene* s, const gy_camera_desc* cam, const gy_s
             if (rc != GY_OK) break;
         }
         // 1. eye pass
-        if (stack64) hipLaunchKernelGGL(k_sppm_eye<64>, dim3(G1(WH, 128)), dim3(128), 0, c->stream, sc->dev, P, D, iter);
-        else hipLaunchKernelGGL(k_sppm_eye<32>, dim3(G1(WH, 128)), dim3(128), 0, c->stream, sc->dev, P, D, iter);
+        if (stack64) hipLaunchKernelGGL(k_sppm_eye<192>, dim3(G1(WH, 128)), dim3(128), 0, c->stream, sc->dev, P, D, iter);
+        else hipLaunchKernelGGL(k_sppm_eye<64>, dim3(G1(WH, 128)), dim3(128), 0, c->stream, sc->dev, P, D, iter);
         rc = CheckLaunch(c, "k_sppm_eye");
         if (rc != GY_OK) break;
         // 2. hash grid

@@ -448,7 +448,7 @@ __device__ V3 vpt_path(const SceneDev& S, const MediaDev& M, const PathParams& P
 template <int STACK, bool ENV, bool EQA>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3)))
 k_vpt(SceneDev S, MediaDev M, PathParams P, FilmDev F, int s0, int n_s) {
-    __shared__ uint32_t stack[STACK * 128];
+    __shared__ uint32_t stack[kPathLds * 128];
     const int64_t t = (int64_t)blockIdx.x * 128 + threadIdx.x;
     int s_local, px, py;
     pass_pixel(F, t, &s_local, &px, &py);
@@ -463,7 +463,7 @@ template <int STACK, bool ENV, bool EQA>
 __global__ void __launch_bounds__(128) k_vpt_li_samples(SceneDev S, MediaDev M, PathParams P, int n, const int32_t* __restrict__ xs,
                                                         const int32_t* __restrict__ ys, const int32_t* __restrict__ ss,
                                                         float* __restrict__ L, float* __restrict__ raster, int32_t* __restrict__ dims) {
-    __shared__ uint32_t stack[STACK * 128];
+    __shared__ uint32_t stack[kPathLds * 128];
     const int i = blockIdx.x * 128 + threadIdx.x;
     if (i >= n) return;
     float fx, fy;
@@ -875,8 +875,8 @@ __device__ inline void vwf_trace_loop(const SceneDev& Sc, const MediaDev& M, con
     const int lane = threadIdx.x & 63;
     const int64_t gl = (int64_t)blockIdx.x * 256 + threadIdx.x;
     uint32_t* lds = stack + threadIdx.x;
-    uint32_t* spill = W.spill + gl;
-    int64_t my = -1;                          // -1 wants work, >= 0 queue index
+    const gyd::SpillGlobal spill{W.spill + gl, W.spill_stride};
+    int32_t my = -1;                          // -1 wants work, >= 0 queue index (below 2^31)
     uint32_t batch_base = 0, batch_left = 0;  // wave-uniform
     bool fresh = false;
     uint32_t slot = 0;
@@ -909,7 +909,7 @@ __device__ inline void vwf_trace_loop(const SceneDev& Sc, const MediaDev& M, con
             const uint32_t rank = (uint32_t)__popcll(nm & ((1ull << lane) - 1ull));
             const uint32_t take = min((uint32_t)__popcll(nm), batch_left);
             if (need && my == -1 && rank < take) {
-                my = batch_base + rank;
+                my = (int32_t)(batch_base + rank);
                 fresh = true;
             }
             batch_base += take;
@@ -936,7 +936,7 @@ __device__ inline void vwf_trace_loop(const SceneDev& Sc, const MediaDev& M, con
                 gyd::trav_init(t, v3f(W.mis_o[slot]), v3f(sd), 0.f, gyd::kInf);
             }
         }
-        if (gyd::trav_run<false, S>(Sc, t, lds, 256, spill, W.spill_stride, refill) == 0) continue;
+        if (gyd::trav_run<false, S>(Sc, t, lds, 256, spill, refill) == 0) continue;
         const bool hit = t.best_prim >= 0;
         bool more = false;  // the lane's segment loop goes on
         if (MODE == 0) {
@@ -1132,18 +1132,18 @@ int LaunchVpt(Ctx* c, Scene* sc, const PathParams& P, int s0, int n_s, bool eqa)
     const int64_t threads = (int64_t)tilesX * tilesY * 64 * n_s;
     const unsigned blocks = (unsigned)((threads + 127) / 128);
     const bool env = sc->dev.env.w > 0;
-    if (sc->stack <= 32) {
-        if (env) LaunchVptT<32, true>(c, sc, P, F, s0, n_s, eqa, blocks);
-        else LaunchVptT<32, false>(c, sc, P, F, s0, n_s, eqa, blocks);
-    } else {
+    if (sc->stack <= 64) {
         if (env) LaunchVptT<64, true>(c, sc, P, F, s0, n_s, eqa, blocks);
         else LaunchVptT<64, false>(c, sc, P, F, s0, n_s, eqa, blocks);
+    } else {
+        if (env) LaunchVptT<192, true>(c, sc, P, F, s0, n_s, eqa, blocks);
+        else LaunchVptT<192, false>(c, sc, P, F, s0, n_s, eqa, blocks);
     }
     return CheckLaunch(c, "k_vpt");
 }
 
 // ---------------------------------------------------------------- wavefront host side
-constexpr int kVwfStack = 16;  // LDS ring entries per lane; deeper stacks spill
+constexpr int kVwfStack = 16;  // LDS stack entries per lane; deeper ones spill
 constexpr int kVwfRefill = 48;
 
 static size_t VwfBytes(int64_t n) {
@@ -1198,7 +1198,7 @@ static int VwfPass(Ctx* c, Scene* sc, const PathParams& P, const FilmDev& F, int
         wf.bytes = VwfBytes(n_slots);
         wf.capacity = n_slots;
     }
-    const size_t sbytes = (size_t)pblocks * 256 * 64 * 4;
+    const size_t sbytes = (size_t)pblocks * 256 * (sc->stack - kVwfStack) * 4;
     if (wf.spill_bytes < sbytes) {
         DevFree(wf.spill);
         wf.spill = nullptr;
@@ -1417,12 +1417,12 @@ extern "C" int gy_vpt_li_samples(gy_scene* s, const gy_camera_desc* cam, const g
     if (rc == GY_OK) {
         const unsigned blocks = (unsigned)((n + 127) / 128);
         const bool env = sc->dev.env.w > 0, eqa = equiangular != 0;
-        auto pick = [&](auto k32, auto k64) { return sc->stack <= 32 ? k32 : k64; };
-        decltype(&k_vpt_li_samples<32, false, false>) kern;
-        if (env) kern = eqa ? pick(k_vpt_li_samples<32, true, true>, k_vpt_li_samples<64, true, true>)
-                            : pick(k_vpt_li_samples<32, true, false>, k_vpt_li_samples<64, true, false>);
-        else kern = eqa ? pick(k_vpt_li_samples<32, false, true>, k_vpt_li_samples<64, false, true>)
-                        : pick(k_vpt_li_samples<32, false, false>, k_vpt_li_samples<64, false, false>);
+        auto pick = [&](auto k32, auto k64) { return sc->stack <= 64 ? k32 : k64; };
+        decltype(&k_vpt_li_samples<64, false, false>) kern;
+        if (env) kern = eqa ? pick(k_vpt_li_samples<64, true, true>, k_vpt_li_samples<192, true, true>)
+                            : pick(k_vpt_li_samples<64, true, false>, k_vpt_li_samples<192, true, false>);
+        else kern = eqa ? pick(k_vpt_li_samples<64, false, true>, k_vpt_li_samples<192, false, true>)
+                        : pick(k_vpt_li_samples<64, false, false>, k_vpt_li_samples<192, false, false>);
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(128), 0, c->stream, sc->dev, MediaView(sc), P, n, (const int32_t*)dx,
                            (const int32_t*)dy, (const int32_t*)ds, (float*)dL, (float*)dr, (int32_t*)dd);
         rc = CheckLaunch(c, "k_vpt_li_samples");

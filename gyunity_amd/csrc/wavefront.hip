@@ -85,7 +85,7 @@ struct WfDev {
     uint32_t sort_blocks;  // ray sort: workgroups of kSortPer queue entries over the capacity
     uint32_t* counts;          // Q_COUNT counters
     int64_t capacity;
-    uint32_t* spill;       // traversal stack spill, 64 entries per lane
+    uint32_t* spill;       // traversal stack entries beyond the LDS part, entry-major
     int64_t spill_stride;  // lanes per launch (grid size)
 };
 
@@ -293,8 +293,8 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
     const int lane = threadIdx.x & 63;
     const int64_t gl = (int64_t)blockIdx.x * 256 + threadIdx.x;
     uint32_t* lds = stack + threadIdx.x;
-    uint32_t* spill = W.spill + gl;
-    int64_t my = -1;  // -1 wants work, -2 queue drained, >= 0 queue index
+    const SpillGlobal spill{W.spill + gl, W.spill_stride};
+    int32_t my = -1;  // -1 wants work, -2 queue drained, >= 0 queue index (a pass holds less than 2^31 paths)
     uint32_t batch_base = 0, batch_left = 0;  // wave-uniform
     bool fresh = false;
     uint32_t slot = 0, e = 0;
@@ -330,7 +330,7 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
             const uint32_t rank = (uint32_t)__popcll(nm & ((1ull << lane) - 1ull));
             const uint32_t take = min((uint32_t)__popcll(nm), batch_left);
             if (need && my == -1 && rank < take) {
-                my = batch_base + rank;
+                my = (int32_t)(batch_base + rank);
                 fresh = true;
             }
             batch_base += take;
@@ -357,7 +357,7 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
                 }
             }
             {
-                const int r = trav_run<kAny, S>(Sc, t, lds, 256, spill, W.spill_stride, refill);
+                const int r = trav_run<kAny, S>(Sc, t, lds, 256, spill, refill);
                 if (r != 0) {
                     if (MODE == 0) {
                         if (t.best_prim >= 0) {
@@ -415,8 +415,10 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
     }
 }
 
+// Six waves per SIMD (80 VGPRs): closest-hit trace of the 1.31M-triangle frame
+// 35.3 ms against 38.7 at five and 40.2 at seven, which spills.
 template <int S, int MODE, class R>
-__global__ void __launch_bounds__(256) k_wf_trace(R Rd, WfDev W, int refill, int chunks) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k_wf_trace(R Rd, WfDev W, int refill, int chunks) {
     __shared__ uint32_t stack[S * 256];
     wf_trace_loop<S, MODE, R>(Rd, W, refill, chunks, stack);
 }
@@ -425,9 +427,11 @@ __global__ void __launch_bounds__(256) k_wf_trace(R Rd, WfDev W, int refill, int
 // shadow queue drained and its lanes idle goes on to the MIS queue while other
 // waves finish their last shadow rays, so the small MIS trace fills the shadow
 // trace's tail instead of running as a launch of its own.  The two kinds set
-// different flag bits of a slot with atomic ORs.
+// different flag bits of a slot with atomic ORs.  Six waves per SIMD as above:
+// 20.9 ms a render against 21.1 at seven, and 1.8 against 2.1 on 3.7M paths
+// under an environment map.
 template <int S, class R>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) k_wf_trace_shadow_mis(R Rd, WfDev W, int refill, int chunks_shadow, int chunks_mis) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k_wf_trace_shadow_mis(R Rd, WfDev W, int refill, int chunks_shadow, int chunks_mis) {
     __shared__ uint32_t stack[S * 256];
     wf_trace_loop<S, 1, R>(Rd, W, refill, chunks_shadow, stack);
     wf_trace_loop<S, 2, R>(Rd, W, refill, chunks_mis, stack);
@@ -963,13 +967,15 @@ static unsigned PersistBlocks(Ctx* c) {
 }
 static int64_t WfLanes(Ctx* c) { return (int64_t)PersistBlocks(c) * 256; }
 
-static int WfPrepareState(Ctx* c, WavefrontState& wf, int64_t n, bool batch) {
-    if (wf.capacity >= n && wf.mem && wf.batch == batch) return GY_OK;
+// `stack`: traversal stack entries a lane can need (Scene::stack); those
+// beyond the LDS part go to the spill buffer.
+static int WfPrepareState(Ctx* c, WavefrontState& wf, int64_t n, bool batch, int stack) {
+    const size_t sbytes = (size_t)WfLanes(c) * (stack - kStackLds) * 4;
+    if (wf.capacity >= n && wf.mem && wf.batch == batch && wf.spill_bytes >= sbytes) return GY_OK;
     WavefrontStateFree(&wf);
     const size_t bytes = WfBytes(n, batch);
     int rc = DevAlloc(c, &wf.mem, bytes);
     if (rc != GY_OK) return rc;
-    const size_t sbytes = (size_t)WfLanes(c) * 64 * 4;
     rc = DevAlloc(c, &wf.spill, sbytes);
     if (rc != GY_OK) return rc;
     wf.capacity = n;
@@ -1057,12 +1063,12 @@ int WavefrontPass(Ctx* c, Scene* sc, const PathParams& P, const gy_render_params
     const int64_t threads = (int64_t)tilesX * tilesY * 64 * n_s;
     const int64_t cap = (int64_t)width * height * n_s;
     if (cap >= (1ll << 31)) return Fail(GY_ERR_UNSUPPORTED, "wavefront pass larger than 2^31 paths");
-    int rc = WfPrepareState(c, sc->wf, std::max<int64_t>(cap, 1), false);
+    int rc = WfPrepareState(c, sc->wf, std::max<int64_t>(cap, 1), false, sc->stack);
     if (rc != GY_OK) return rc;
     size_t used = 0;
     WfDev W = g_view(sc->wf, false, &used);
     W.spill_stride = WfLanes(c);
-    if ((size_t)W.spill_stride * 64 * 4 > sc->wf.spill_bytes) return Fail(GY_ERR_ALLOC, "wavefront spill buffer too small");
+    if ((size_t)W.spill_stride * (sc->stack - kStackLds) * 4 > sc->wf.spill_bytes) return Fail(GY_ERR_ALLOC, "wavefront spill buffer too small");
     if (used > sc->wf.bytes) return Fail(GY_ERR_ALLOC, "wavefront state layout exceeds its allocation");
     OneRender Rd;
     Rd.S = sc->dev;
@@ -1229,12 +1235,12 @@ __global__ void __launch_bounds__(256) k_lt_shade(SceneDev S, PathParams P, WfDe
 
 int LightTracingWavefront(Ctx* c, Scene* sc, const PathParams& P, const LightCamDev& C, int64_t n, float total, float* splat) {
     const int64_t cap = std::min<int64_t>(n, (int64_t)1 << 26);
-    int rc = WfPrepareState(c, sc->wf, std::max<int64_t>(cap, 1), false);
+    int rc = WfPrepareState(c, sc->wf, std::max<int64_t>(cap, 1), false, sc->stack);
     if (rc != GY_OK) return rc;
     size_t used = 0;
     WfDev W = g_view(sc->wf, false, &used);
     W.spill_stride = WfLanes(c);
-    if ((size_t)W.spill_stride * 64 * 4 > sc->wf.spill_bytes) return Fail(GY_ERR_ALLOC, "wavefront spill buffer too small");
+    if ((size_t)W.spill_stride * (sc->stack - kStackLds) * 4 > sc->wf.spill_bytes) return Fail(GY_ERR_ALLOC, "wavefront spill buffer too small");
     if (used > sc->wf.bytes) return Fail(GY_ERR_ALLOC, "wavefront state layout exceeds its allocation");
     LightRender Rd;
     Rd.S = sc->dev;
@@ -1293,7 +1299,6 @@ static int BatchSequence(Ctx* c, Batch* b) {
     size_t used = 0;
     WfDev W = g_view(b->wf, true, &used);
     W.spill_stride = WfLanes(c);
-    if ((size_t)W.spill_stride * 64 * 4 > b->wf.spill_bytes) return Fail(GY_ERR_ALLOC, "wavefront spill buffer too small");
     if (used > b->wf.bytes) return Fail(GY_ERR_ALLOC, "wavefront state layout exceeds its allocation");
     ManyRenders Rd;
     Rd.E = (const BatchEntryDev*)b->table;
@@ -1323,7 +1328,9 @@ static int BatchSequence(Ctx* c, Batch* b) {
 }
 
 int BatchRender(Ctx* c, Batch* b) {
-    int rc = WfPrepareState(c, b->wf, b->lanes, true);
+    int stack = kStackSmall;
+    for (const BatchEntry& en : b->entries) stack = std::max(stack, en.scene->stack);
+    int rc = WfPrepareState(c, b->wf, b->lanes, true, stack);
     if (rc != GY_OK) return rc;
     if (!b->use_graph) return BatchSequence(c, b);
     if (!b->graph_exec) {
