@@ -63,6 +63,13 @@ GY_D V3 ld3(const float4 q) { return V3{q.x, q.y, q.z}; }
 // in the last ulp).
 GY_D float dcos(float x) { return (float)cos((double)x); }
 GY_D float dsin(float x) { return (float)sin((double)x); }
+// Both at once: one argument reduction in place of two.
+GY_D void dsincos(float x, float* s, float* c) {
+    double ds, dc;
+    sincos((double)x, &ds, &dc);
+    *s = (float)ds;
+    *c = (float)dc;
+}
 GY_D float dlog(float x) { return (float)log((double)x); }
 GY_D float dacos(float x) { return (float)acos((double)x); }
 GY_D float datan2(float y, float x) { return (float)atan2((double)y, (double)x); }
@@ -787,8 +794,10 @@ GY_D V3 cosine_hemisphere(float u0, float u1) {
             r = oy;
             theta = kPIOver2 - kPIOver4 * (ox / oy);
         }
-        dx = r * dcos(theta);
-        dy = r * dsin(theta);
+        float st, ct;
+        dsincos(theta, &st, &ct);
+        dx = r * ct;
+        dy = r * st;
     }
     const float z = sqrtf(rmax(0.f, 1 - dx * dx - dy * dy));
     return v3(dx, dy, z);
@@ -853,8 +862,10 @@ GY_D V3 ggx_sample_wh(const GGX& g, V3 v_, float u0, float u1) {
     const float a = 1.f / (1.f + v.z);
     const float r = sqrtf(u0);
     const float phi = (u1 < a) ? u1 / a * kPI : kPI + (u1 - a) / (1.f - a) * kPI;
-    const float P1 = r * dcos(phi);
-    const float P2 = r * dsin(phi) * ((u1 < a) ? 1.0f : v.z);
+    float sphi, cphi;
+    dsincos(phi, &sphi, &cphi);
+    const float P1 = r * cphi;
+    const float P2 = r * sphi * ((u1 < a) ? 1.0f : v.z);
     const V3 dir = (P1 * T1 + P2 * T2) + sqrtf(rmax(0.f, 1 - P1 * P1 - P2 * P2)) * v;
     return norm(v3(g.ax * dir.x, g.ay * dir.y, rmax(0.f, dir.z)));
 }
@@ -1220,7 +1231,8 @@ __device__ __noinline__ LightPoint sph_sample_li(const SceneDev& S, int i, V3 re
     const float sdist = dis * cosTheta - sqrtf(rmax(rad * rad - dis * dis * sinTheta * sinTheta, 0.f));
     const float cosAlpha = (dis * dis + rad * rad - sdist * sdist) / (2 * dis * rad);
     const float sinAlpha = sqrtf(rmax(1.f - cosAlpha * cosAlpha, 0.f));
-    const float cphi = dcos(phi), sphi = dsin(phi);
+    float sphi, cphi;
+    dsincos(phi, &sphi, &cphi);
     V3 nWorld = ((-1.f * sinAlpha * cphi) * localX - (sinAlpha * sphi) * localY) - cosAlpha * localZ;
     nWorld = norm(nWorld);
     const float off = (float)((double)rad * 1.5e-3);
@@ -1324,8 +1336,10 @@ GY_D void env_dir_to_uv(V3 d, float* u, float* v) {
 GY_D V3 env_uv_to_dir(float u, float v) {
     const float phi = u * 2 * kPI;
     const float theta = v * kPI;
-    const float st = dsin(theta);
-    return v3(st * dcos(phi), dcos(theta), st * dsin(phi));
+    float st, ct, sp, cp;
+    dsincos(theta, &st, &ct);
+    dsincos(phi, &sp, &cp);
+    return v3(st * cp, ct, st * sp);
 }
 // SinTheta (light/EnvMap.h:124-132).
 GY_D float env_sin_theta(float v, float height) {

@@ -358,7 +358,8 @@ __device__ inline void film_footprint(float fx, float fy, int W, int H, int* x0,
 // footprint beyond the neighbouring pixels is counted in F.border[W * H] and
 // fails the render.
 constexpr uint32_t kFilmOwn = 1u << 4;
-__device__ inline void film_record(const FilmDev& F, int64_t slot, int px, int py, float fx, float fy, V3 L) {
+// The footprint mask of a sample, its pixel's border flag and the error count.
+__device__ inline uint32_t film_mark(const FilmDev& F, int px, int py, float fx, float fy) {
     const int W = F.width, H = F.height;
     int x0, x1, y0, y1;
     film_footprint(fx, fy, W, H, &x0, &x1, &y0, &y1);
@@ -374,9 +375,12 @@ __device__ inline void film_record(const FilmDev& F, int64_t slot, int px, int p
             if (dx < -1 || dx > 1 || dy < -1 || dy > 1) far = true;
             else mask |= 1u << ((dy + 1) * 3 + dx + 1);
         }
-    F.pass[slot] = make_float4(L.x, L.y, L.z, (float)mask);
     if (mask != kFilmOwn) F.border[(int64_t)py * W + px] = 1u;
     if (far) atomicAdd(F.border + (int64_t)W * H, 1u);
+    return mask;
+}
+__device__ inline void film_record(const FilmDev& F, int64_t slot, int px, int py, float fx, float fy, V3 L) {
+    F.pass[slot] = make_float4(L.x, L.y, L.z, (float)film_mark(F, px, py, fx, fy));
 }
 
 __device__ inline void record_sample(const FilmDev& F, int s_local, int px, int py, float fx, float fy, V3 L) {

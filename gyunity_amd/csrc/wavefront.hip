@@ -45,11 +45,19 @@ constexpr int C_WORDS = 48;
 // queues do not serialise on one L2 channel.
 constexpr int kCtrStride = 32;
 
-// Path flags (PathState.seq.w)
-constexpr uint32_t F_DEPTH_MASK = 0xffu;
-constexpr uint32_t F_DELTA = 1u << 8;
-// Resolve flags (pend3.w as bits): pending direct light of this bounce, and the
-// path's end.  Zero for a slot with nothing to resolve.
+// Path state word (T.w): sample dimensions drawn (at most 2 + 100 * 10), depth
+// (at most 100), whether the last bounce was a delta one, and the film footprint
+// mask of the path's sample (film_mark).
+constexpr uint32_t kStCursor = 0x7ffu;
+constexpr int kStDepth = 11;  // 7 bits
+constexpr uint32_t kStDepthMask = 0x7fu;
+constexpr uint32_t kStDelta = 1u << 18;
+constexpr int kStMask = 19;  // 9 bits
+__device__ inline uint32_t st_pack(uint32_t cursor, uint32_t depth, bool delta, uint32_t mask) {
+    return cursor | (depth << kStDepth) | (delta ? kStDelta : 0u) | (mask << kStMask);
+}
+// Resolve flags: pending direct light of this bounce, and the path's end.  Zero
+// for a slot with nothing to resolve.
 constexpr uint32_t P_HAS_DI = 1u;
 constexpr uint32_t P_OCCLUDED = 2u;
 constexpr uint32_t P_L2 = 4u;
@@ -58,24 +66,40 @@ constexpr uint32_t P_W2_NF = 16u;  // w2 not finite: 0 * w2 is NaN
 constexpr uint32_t P_DONE = 32u;   // the path ended this bounce: it goes to the film
 constexpr uint32_t P_NEXT = 64u;   // the path goes on without pending direct light
 constexpr uint32_t P_ESC = 128u;   // the MIS ray left the scene (k_wf_env adds an environment light's L2)
+constexpr uint32_t P_FULL = 256u;  // the direct light is in pend0-2 and pT, not in C
 // A path goes on after this bounce iff its flags are non-zero without P_DONE.
 
+// Path state, one array per record (structure of arrays).  Shading and
+// resolving are bound by the bytes they move (128 bytes written a shading point
+// and 2.6 TB/s when every record was 16 bytes wide; fewer loads, from LDS tables
+// of the Sobol samples, or more waves changed nothing), so vectors are 12 bytes,
+// what does not change over a path (its sample index, its footprint) is written
+// once, the state shares the throughput's record, and the direct light of a
+// path without an MIS ray is one vector, added when its shadow ray got through:
+// 84 bytes.  1.31M triangles, 67M paths: shading 45.0 -> 34.4 ms a render,
+// resolving and binning 14.8 -> 11.5.
+struct HitRec {
+    int32_t prim;
+    float b1, b2;
+};
 struct WfDev {
-    float4* o;      // ray origin (xyz)
-    float4* d;      // ray direction (xyz)
-    float4* T;      // throughput (xyz), film x in w
-    float4* L;      // radiance (xyz), film y in w
-    uint4* seq;     // sample index lo/hi, cursor, flags
-    float4* hit;    // t, prim, b1, b2
-    uint8_t* mtype;  // per slot: material type of the closest hit (0..3), 255 for a miss
-    float4* pend0;  // L1 w1 before the shadow test (xyz), P(light)
-    float4* pend1;  // MIS ray only: BSDF value of the MIS sample (xyz) / L2 w2 after trace_mis, cos
-    float4* pend2;  // MIS ray only: pdf of the MIS sample, w2, -, light id
-    float4* pend3;  // throughput at this bounce (xyz), resolve flags (P_*)
+    V3* o;          // ray origin
+    V3* d;          // ray direction
+    float4* T;      // throughput (xyz), state word
+    V3* L;          // radiance
+    uint2* idx;     // sample index
+    HitRec* hit;
+    uint8_t* mtype;   // per slot: material type of the closest hit (0..3), 255 for a miss
+    uint32_t* flags;  // resolve flags (P_*)
+    V3* C;            // direct light: T (L1 w1 + 0) / P(light), to add unless occluded
+    float4* pend0;  // full record: L1 w1 before the shadow test (xyz), P(light); light tracing: a connection's splat, pixel
+    float4* pend1;  // full record: BSDF value of the MIS sample (xyz) / L2 w2 after trace_mis, cos
+    float4* pend2;  // full record: pdf of the MIS sample, w2, -, light id
+    V3* pT;         // full record: throughput at this bounce
     float4* sh_o;   // shadow ray origin, tmax
-    float4* sh_d;   // shadow ray direction
-    float4* mis_o;  // MIS ray origin
-    float4* mis_d;  // MIS ray direction
+    V3* sh_d;       // shadow ray direction
+    V3* mis_o;      // MIS ray origin
+    V3* mis_d;      // MIS ray direction
     uint32_t* ent;    // batch: entry of the lane
     uint32_t* pslot;  // batch: the path's slot in its entry's pass buffer
     uint32_t* q[Q_COUNT];  // Q_ACTIVE, Q_NEXT, 4 shade queues, shadow, mis
@@ -184,7 +208,7 @@ __device__ inline V3 f3(const float4 v) { return v3(v.x, v.y, v.z); }
 
 // Camera sample of one path (TiledIntegrator::Render per sample,
 // integrator/TiledIntegrator.cpp:40-45) into lane `slot`.
-__device__ inline void start_path(const WfDev& W, const PathParams& P, uint32_t slot, int s, int px, int py) {
+__device__ inline void start_path(const WfDev& W, const PathParams& P, const FilmDev& F, uint32_t slot, int s, int px, int py) {
     Seq q;
     q.index = enum_index(P.en, (uint32_t)s, (uint32_t)px, (uint32_t)py);
     q.cursor = 0;
@@ -192,18 +216,20 @@ __device__ inline void start_path(const WfDev& W, const PathParams& P, uint32_t 
     const float v = P.en.sy * seq_next_wide(P.smp, q) - (float)py;
     V3 o, d;
     generate_ray(P.cam, px, py, u, v, &o, &d);
-    W.o[slot] = make_float4(o.x, o.y, o.z, 0.f);
-    W.d[slot] = make_float4(d.x, d.y, d.z, 0.f);
-    W.T[slot] = make_float4(1.f, 1.f, 1.f, px + u);
-    W.L[slot] = make_float4(0.f, 0.f, 0.f, py + v);
-    W.seq[slot] = make_uint4((uint32_t)q.index, (uint32_t)(q.index >> 32), q.cursor, 0u);
-    W.pend3[slot] = make_float4(0.f, 0.f, 0.f, __uint_as_float(P.max_depth == 0 ? P_DONE : 0u));
+    const uint32_t mask = film_mark(F, px, py, px + u, py + v);
+    W.o[slot] = o;
+    W.d[slot] = d;
+    W.T[slot] = make_float4(1.f, 1.f, 1.f, __uint_as_float(st_pack(q.cursor, 0u, false, mask)));
+    W.L[slot] = v3s(0.f);
+    W.idx[slot] = make_uint2((uint32_t)q.index, (uint32_t)(q.index >> 32));
+    W.flags[slot] = P.max_depth == 0 ? P_DONE : 0u;
 }
 
 // ---------------------------------------------------------------- raygen
 // One render: samples s0 .. s0+n_s-1 of every pixel, 8x8 pixel tiles per wave.
-__global__ void __launch_bounds__(256) k_wf_raygen(WfDev W, PathParams P, int s0, int n_s, int width, int height) {
+__global__ void __launch_bounds__(256) k_wf_raygen(WfDev W, PathParams P, FilmDev F, int s0, int n_s) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int width = F.width, height = F.height;
     const int tilesX = (width + 7) >> 3, tilesY = (height + 7) >> 3;
     const int64_t per_s = (int64_t)tilesX * tilesY * 64;
     bool valid = t < per_s * n_s;
@@ -218,7 +244,7 @@ __global__ void __launch_bounds__(256) k_wf_raygen(WfDev W, PathParams P, int s0
         valid = px < width && py < height;
     }
     const uint32_t slot = (uint32_t)((int64_t)s_local * width * height + (int64_t)py * width + px);
-    if (valid) start_path(W, P, slot, s0 + s_local, px, py);
+    if (valid) start_path(W, P, F, slot, s0 + s_local, px, py);
     uint32_t* const qa[1] = {W.q[Q_ACTIVE]};
     uint32_t* const ca[1] = {&W.counts[Q_ACTIVE * kCtrStride]};
     const bool pa[1] = {valid};
@@ -258,9 +284,9 @@ __global__ void __launch_bounds__(256) k_wf_raygen_batch(WfDev W, ManyRenders R,
         const PathParams& P = R.E[e].P;
         W.ent[slot] = e;
         W.pslot[slot] = (uint32_t)((int64_t)s * P.cam.width * P.cam.height + (int64_t)py * P.cam.width + px);
-        start_path(W, P, slot, s, px, py);
+        start_path(W, P, R.E[e].F, slot, s, px, py);
     } else if (t < lanes) {
-        W.pend3[slot].w = __uint_as_float(0u);  // resolve walks every lane: one without a path has no flags
+        W.flags[slot] = 0u;  // resolve walks every lane: one without a path has no flags
     }
     uint32_t* const qa[1] = {W.q[Q_ACTIVE]};
     uint32_t* const ca[1] = {&W.counts[Q_ACTIVE * kCtrStride]};
@@ -348,12 +374,12 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
                     Sc.tri = Rd.scene(e).tri;
                 }
                 if (MODE == 0) {
-                    trav_init(t, f3(W.o[slot]), f3(W.d[slot]), 0.f, kInf);
+                    trav_init(t, W.o[slot], W.d[slot], 0.f, kInf);
                 } else if (kAny) {
                     const float4 o = W.sh_o[slot];
-                    trav_init(t, f3(o), f3(W.sh_d[slot]), 0.f, o.w);
+                    trav_init(t, f3(o), W.sh_d[slot], 0.f, o.w);
                 } else {
-                    trav_init(t, f3(W.mis_o[slot]), f3(W.mis_d[slot]), 0.f, kInf);
+                    trav_init(t, W.mis_o[slot], W.mis_d[slot], 0.f, kInf);
                 }
             }
             {
@@ -362,16 +388,16 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
                     if (MODE == 0) {
                         if (t.best_prim >= 0) {
                             const SceneDev& Sf = Rd.scene(e);
-                            W.hit[slot] = make_float4(t.best, __int_as_float(t.best_prim), t.bb1, t.bb2);
+                            W.hit[slot] = HitRec{t.best_prim, t.bb1, t.bb2};
                             const uint32_t mat = __float_as_uint(Sf.shade[(size_t)t.best_prim * 8].w);
                             W.mtype[slot] = (uint8_t)Sf.mats[(size_t)mat * 32];
                         } else {
                             W.mtype[slot] = 255;
-                            W.pend3[slot].w = __uint_as_float(P_DONE);  // the path ends (k_wf_env: environment)
+                            W.flags[slot] = P_DONE;  // the path ends (k_wf_env: environment)
                         }
                     } else if (MODE == 1) {
                         // atomic: the slot's MIS ray may be in flight in the same launch
-                        if (r == 2) atomicOr(reinterpret_cast<uint32_t*>(&W.pend3[slot].w), P_OCCLUDED);
+                        if (r == 2) atomicOr(&W.flags[slot], P_OCCLUDED);
                     } else if (MODE == 3) {
                         if constexpr (MODE == 3) {
                             // Film::AddSplat (visual/Film.h:89-103) of an unoccluded connection
@@ -385,7 +411,7 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
                         }
                     } else if (t.best_prim < 0) {
                         // a miss counts for an environment light (k_wf_env)
-                        if (Rd.scene(e).env.w > 0) atomicOr(reinterpret_cast<uint32_t*>(&W.pend3[slot].w), P_ESC);
+                        if (Rd.scene(e).env.w > 0) atomicOr(&W.flags[slot], P_ESC);
                     } else {
                         // MIS branch of DirectIllumination (integrator/Integrator.cpp:88-98)
                         const SceneDev& Sf = Rd.scene(e);
@@ -405,7 +431,7 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
                             const V3 L2 = Lem * f3(p1) * v3s(1.f) * p1.w / p2.x;
                             const V3 L2w2 = L2 * p2.y;
                             W.pend1[slot] = make_float4(L2w2.x, L2w2.y, L2w2.z, p1.w);
-                            atomicOr(reinterpret_cast<uint32_t*>(&W.pend3[slot].w), P_L2);
+                            atomicOr(&W.flags[slot], P_L2);
                         }
                     }
                     my = -1;
@@ -453,7 +479,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 // offset + rank in the workgroup).
 constexpr int kSortPer = 1024;  // queue entries per workgroup, 4 per thread
 
-__device__ inline uint32_t ray_octant(const float4 d) {
+__device__ inline uint32_t ray_octant(const V3 d) {
     return (__float_as_uint(d.x) >> 31) | ((__float_as_uint(d.y) >> 31) << 1) | ((__float_as_uint(d.z) >> 31) << 2);
 }
 
@@ -647,22 +673,20 @@ __global__ void __launch_bounds__(256) k_wf_env(R Rd, WfDev W) {
     if (S.env.w == 0) return;
     if (MODE == 0) {
         if (W.mtype[slot] != 255) return;
-        const uint32_t sw = W.seq[slot].w;
-        if ((sw & F_DEPTH_MASK) != 0u && !(sw & F_DELTA)) return;
-        const float4 Lv = W.L[slot];
-        const V3 L = f3(W.T[slot]) * env_emission(S.env, f3(W.d[slot]));
-        W.L[slot] = make_float4(L.x, L.y, L.z, Lv.w);
+        const float4 Tv = W.T[slot];
+        const uint32_t st = __float_as_uint(Tv.w);
+        if (((st >> kStDepth) & kStDepthMask) != 0u && !(st & kStDelta)) return;
+        W.L[slot] = f3(Tv) * env_emission(S.env, W.d[slot]);
     } else {
-        float& fw = W.pend3[slot].w;
-        const uint32_t pf = __float_as_uint(fw);
+        const uint32_t pf = W.flags[slot];
         if (!(pf & P_ESC)) return;
         const float4 p2 = W.pend2[slot];
         if (S.light_tri[__float_as_int(p2.w)] >= 0) return;
         const float4 p1 = W.pend1[slot];
-        const V3 L2 = env_emission(S.env, f3(W.mis_d[slot])) * f3(p1) * v3s(1.f) * p1.w / p2.x;
+        const V3 L2 = env_emission(S.env, W.mis_d[slot]) * f3(p1) * v3s(1.f) * p1.w / p2.x;
         const V3 L2w2 = L2 * p2.y;
         W.pend1[slot] = make_float4(L2w2.x, L2w2.y, L2w2.z, p1.w);
-        fw = __uint_as_float(pf | P_L2);
+        W.flags[slot] = pf | P_L2;
     }
 }
 
@@ -683,20 +707,21 @@ __global__ void __launch_bounds__(256) k_wf_shade(R Rd, WfDev W) {
         const SceneDev& S = Rd.scene(e);
         const PathParams& P = Rd.params(e);
         const SampleSrc& M = P.smp;
-        const V3 ro = f3(W.o[slot]), rd = f3(W.d[slot]);
-        const float4 hv = W.hit[slot];
-        Hit h;
-        h.t = hv.x;
-        h.prim = __float_as_int(hv.y);
-        h.b1 = hv.z;
-        h.b2 = hv.w;
-        uint4 sq = W.seq[slot];
-        Seq q;
-        q.index = (uint64_t)sq.x | ((uint64_t)sq.y << 32);
-        q.cursor = sq.z;
-        const int depth = (int)(sq.w & F_DEPTH_MASK);
-        const bool delta = (sq.w & F_DELTA) != 0;
+        const V3 ro = W.o[slot], rd = W.d[slot];
         const float4 Tv = W.T[slot];
+        const uint32_t st = __float_as_uint(Tv.w);
+        const HitRec hv = W.hit[slot];
+        Hit h;
+        h.t = 0.f;  // not read
+        h.prim = hv.prim;
+        h.b1 = hv.b1;
+        h.b2 = hv.b2;
+        const uint2 ix = W.idx[slot];
+        Seq q;
+        q.index = (uint64_t)ix.x | ((uint64_t)ix.y << 32);
+        q.cursor = st & kStCursor;
+        const int depth = (int)((st >> kStDepth) & kStDepthMask);
+        const bool delta = (st & kStDelta) != 0;
         V3 T = f3(Tv);
         const Isect it = query(S, ro, rd, h);
         BSDF b = make_bsdf(S, it);
@@ -706,9 +731,7 @@ __global__ void __launch_bounds__(256) k_wf_shade(R Rd, WfDev W) {
             const V3 Le = v3(S.light_le[3 * it.light], S.light_le[3 * it.light + 1], S.light_le[3 * it.light + 2]);
             const V3 em = dot(it.n, it.outDir) > 0.f ? Le : v3(0.f, 0.f, 0.f);
             // radiance changes only here: read and written on this branch alone
-            const float4 Lv = W.L[slot];
-            const V3 L = f3(Lv) + T * em;
-            W.L[slot] = make_float4(L.x, L.y, L.z, Lv.w);
+            W.L[slot] = W.L[slot] + T * em;
         } else {
             const float uL = seq_next_wide(M, q);
             const float u0 = seq_next_wide(M, q), u1 = seq_next_wide(M, q);
@@ -740,7 +763,7 @@ __global__ void __launch_bounds__(256) k_wf_shade(R Rd, WfDev W) {
                         float stmax;
                         spawn_to(it, lp, &so, &sd, &stmax);
                         W.sh_o[slot] = make_float4(so.x, so.y, so.z, stmax);
-                        W.sh_d[slot] = make_float4(sd.x, sd.y, sd.z, 0.f);
+                        W.sh_d[slot] = sd;
                         push_shadow = true;
                         w1 = power_heuristic(pdf, sp);
                         L1pre = Li * v3s(1.f) * f * c / pdf;
@@ -759,8 +782,8 @@ __global__ void __launch_bounds__(256) k_wf_shade(R Rd, WfDev W) {
                     w2 = power_heuristic(pdf2, lpdf);
                     V3 mo;
                     spawn_ray(it, wi2, &mo);
-                    W.mis_o[slot] = make_float4(mo.x, mo.y, mo.z, 0.f);
-                    W.mis_d[slot] = make_float4(wi2.x, wi2.y, wi2.z, 0.f);
+                    W.mis_o[slot] = mo;
+                    W.mis_d[slot] = wi2;
                     push_mis = true;
                 }
             }
@@ -768,20 +791,28 @@ __global__ void __launch_bounds__(256) k_wf_shade(R Rd, WfDev W) {
             // of DirectIllumination are formed in the same FP32 operations,
             // and a zero L1 (occluded) or L2 (no MIS ray) gives +0 for them, as
             // 0 * w does for a finite weight (NaN for an infinite or NaN one,
-            // flagged below).  The MIS records are written only for a path
-            // that has an MIS ray.
+            // flagged below).  Few paths have an MIS ray (its direction has to
+            // hit the chosen light).  Without one and with finite factors the
+            // light is L += T (L1 w1 + 0) / P(light) if the shadow ray gets
+            // through, and L += +-0, which changes no sum that started from
+            // +0, if it does not or if there is none.
             const V3 L1w1 = L1pre * w1;
-            W.pend0[slot] = make_float4(L1w1.x, L1w1.y, L1w1.z, lsp);
-            if (push_mis) {
+            const bool full = push_mis || !(isfinite(w1) && isfinite(w2) && isfinite(lsp) && isfinite(T.x) &&
+                                            isfinite(T.y) && isfinite(T.z));
+            if (full) {
+                W.pend0[slot] = make_float4(L1w1.x, L1w1.y, L1w1.z, lsp);
                 W.pend1[slot] = make_float4(f2.x, f2.y, f2.z, c2);
                 W.pend2[slot] = make_float4(pdf2, w2, lsp, __int_as_float(light));
+                W.pT[slot] = T;
+                pflags = P_HAS_DI | P_FULL | (isfinite(w1) ? 0u : P_W1_NF) | (isfinite(w2) ? 0u : P_W2_NF);
+            } else if (push_shadow) {
+                W.C[slot] = T * ((L1w1 + v3s(0.f)) / lsp);
+                pflags = P_HAS_DI;
             }
-            pflags = P_HAS_DI | (isfinite(w1) ? 0u : P_W1_NF) | (isfinite(w2) ? 0u : P_W2_NF);
-            W.pend3[slot] = make_float4(T.x, T.y, T.z, __uint_as_float(pflags));
         }
         // BSDF continuation and Russian roulette (integrator/PT.cpp:45-62)
         bool alive = depth + 1 < P.max_depth;
-        uint32_t nflags = sq.w;
+        uint32_t nst = 0;
         if (alive) {
             const float r0 = seq_next_wide(M, q), r1 = seq_next_wide(M, q), r2 = seq_next_wide(M, q);
             V3 wi;
@@ -801,20 +832,15 @@ __global__ void __launch_bounds__(256) k_wf_shade(R Rd, WfDev W) {
                     T = T * est;
                     V3 o;
                     spawn_ray(it, wi, &o);
-                    W.o[slot] = make_float4(o.x, o.y, o.z, 0.f);
-                    W.d[slot] = make_float4(wi.x, wi.y, wi.z, 0.f);
-                    nflags = (nflags & ~(F_DEPTH_MASK | F_DELTA)) | (uint32_t)(depth + 1) | (ndelta ? F_DELTA : 0u);
+                    W.o[slot] = o;
+                    W.d[slot] = wi;
+                    nst = st_pack(q.cursor, (uint32_t)(depth + 1), ndelta, st >> kStMask);
                 }
             }
         }
-        if (alive) {  // a path that ends keeps T unchanged and needs no sample state
-            W.T[slot] = make_float4(T.x, T.y, T.z, Tv.w);
-            W.seq[slot] = make_uint4(sq.x, sq.y, q.cursor, nflags);
-        }
-        // the flags word: written with the pending record above for a path that
-        // goes on; otherwise here (a path that ends, or one without direct light
-        // whose flags still hold the last bounce's)
-        if (!alive || !(pflags & P_HAS_DI)) W.pend3[slot].w = __uint_as_float(alive ? P_NEXT : (pflags | P_DONE));
+        // a path that ends keeps T and its state
+        if (alive) W.T[slot] = make_float4(T.x, T.y, T.z, __uint_as_float(nst));
+        W.flags[slot] = alive ? (pflags ? pflags : P_NEXT) : (pflags | P_DONE);
     }
     uint32_t* const qs[2] = {W.q[Q_SHADOW], W.q[Q_MIS]};
     uint32_t* const cs[2] = {&W.counts[Q_SHADOW * kCtrStride], &W.counts[Q_MIS * kCtrStride]};
@@ -828,32 +854,34 @@ __global__ void __launch_bounds__(256) k_wf_shade(R Rd, WfDev W) {
 // form the next bounce's active queue.  Returns whether the path goes on.
 template <class R>
 __device__ inline bool resolve_slot(const R& Rd, const WfDev& W, uint32_t slot) {
-    const float4 p3 = W.pend3[slot];
-    const uint32_t pf = __float_as_uint(p3.w);
+    const uint32_t pf = W.flags[slot];
     if (pf == 0u) return false;  // no path in the slot
     const bool done = (pf & P_DONE) != 0u;
-    if (!(pf & P_HAS_DI) && !done) return true;
-    float4 Lv = W.L[slot];
-    if (pf & P_HAS_DI) {
-        const float4 p0 = W.pend0[slot];
-        const float nan = __builtin_nanf("");
-        const V3 L1w1 = (pf & P_OCCLUDED) ? v3s((pf & P_W1_NF) ? nan : 0.f) : f3(p0);
-        const V3 L2w2 = (pf & P_L2) ? f3(W.pend1[slot]) : v3s((pf & P_W2_NF) ? nan : 0.f);
-        const V3 DI = (L1w1 + L2w2) / p0.w;
-        const V3 L = f3(Lv) + f3(p3) * DI;
-        Lv = make_float4(L.x, L.y, L.z, Lv.w);
+    // an occluded light without a full record leaves L as it is
+    const bool add = (pf & P_HAS_DI) != 0u && (pf & (P_FULL | P_OCCLUDED)) != P_OCCLUDED;
+    if (!add && !done) return true;
+    V3 L = W.L[slot];
+    if (add) {
+        if (pf & P_FULL) {
+            const float4 p0 = W.pend0[slot];
+            const float nan = __builtin_nanf("");
+            const V3 L1w1 = (pf & P_OCCLUDED) ? v3s((pf & P_W1_NF) ? nan : 0.f) : f3(p0);
+            const V3 L2w2 = (pf & P_L2) ? f3(W.pend1[slot]) : v3s((pf & P_W2_NF) ? nan : 0.f);
+            L = L + W.pT[slot] * ((L1w1 + L2w2) / p0.w);
+        } else {
+            L = L + W.C[slot];
+        }
         if (!done) {
-            W.L[slot] = Lv;
+            W.L[slot] = L;
             return true;
         }
     }
-    W.pend3[slot].w = __uint_as_float(0u);  // resolved: later bounces skip the slot
-    // Film::AddSample (visual/Film.h:61-87) through the pass buffer
+    W.flags[slot] = 0u;  // resolved: later bounces skip the slot
+    // Film::AddSample (visual/Film.h:61-87) through the pass buffer; raygen has
+    // marked the sample's footprint (film_mark)
     const FilmDev& F = Rd.film(Rd.entry(W, slot));
     const uint32_t ps = Rd.pass_slot(W, slot);
-    const int64_t WH = (int64_t)F.width * F.height;
-    const int64_t pix = ps % WH;
-    film_record(F, ps, (int)(pix % F.width), (int)(pix / F.width), W.T[slot].w, Lv.w, v3(Lv.x, Lv.y, Lv.z));
+    F.pass[ps] = make_float4(L.x, L.y, L.z, (float)(__float_as_uint(W.T[slot].w) >> kStMask));
     return false;
 }
 
@@ -862,7 +890,7 @@ __device__ inline bool resolve_slot(const R& Rd, const WfDev& W, uint32_t slot) 
 // order the queues left the paths in, and the next active queue comes out in
 // slot order: shading, which works through queues, then reads and writes the
 // path records of neighbouring slots together.  A slot with no flags costs one
-// 16-byte load.  A path that goes on keeps its flags, which the next bounce
+// 4-byte load.  A path that goes on keeps its flags, which the next bounce
 // rewrites (shading, or the closest-hit miss) before they are read again.
 constexpr int kResolvePerThread = 4;
 template <class R>
@@ -904,21 +932,23 @@ static WfDev g_view(const WavefrontState& wf, bool batch, size_t* used) {
         off += (bytes + 255) & ~(size_t)255;
         return p;
     };
-    W.o = (float4*)take(n * 16);
-    W.d = (float4*)take(n * 16);
+    W.o = (V3*)take(n * 12);
+    W.d = (V3*)take(n * 12);
     W.T = (float4*)take(n * 16);
-    W.L = (float4*)take(n * 16);
-    W.seq = (uint4*)take(n * 16);
-    W.hit = (float4*)take(n * 16);
+    W.L = (V3*)take(n * 12);
+    W.idx = (uint2*)take(n * 8);
+    W.hit = (HitRec*)take(n * 12);
     W.mtype = (uint8_t*)take(n);
+    W.flags = (uint32_t*)take(n * 4);
+    W.C = (V3*)take(n * 12);
     W.pend0 = (float4*)take(n * 16);
     W.pend1 = (float4*)take(n * 16);
     W.pend2 = (float4*)take(n * 16);
-    W.pend3 = (float4*)take(n * 16);
+    W.pT = (V3*)take(n * 12);
     W.sh_o = (float4*)take(n * 16);
-    W.sh_d = (float4*)take(n * 16);
-    W.mis_o = (float4*)take(n * 16);
-    W.mis_d = (float4*)take(n * 16);
+    W.sh_d = (V3*)take(n * 12);
+    W.mis_o = (V3*)take(n * 12);
+    W.mis_d = (V3*)take(n * 12);
     W.ent = batch ? (uint32_t*)take(n * 4) : nullptr;
     W.pslot = batch ? (uint32_t*)take(n * 4) : nullptr;
     for (int q = 0; q < Q_COUNT; ++q) W.q[q] = (uint32_t*)take(n * 4);
@@ -935,9 +965,9 @@ static WfDev g_view(const WavefrontState& wf, bool batch, size_t* used) {
 }
 
 static size_t WfBytes(int64_t n, bool batch) {
-    const size_t per = 14 * 16 + 1 + (Q_COUNT + 1) * 4 + (batch ? 8 : 0);
+    const size_t per = 5 * 16 + 9 * 12 + 8 + 4 + 1 + (Q_COUNT + 1) * 4 + (batch ? 8 : 0);
     const size_t hist = ((size_t)((n + kSortPer - 1) / kSortPer) * 8 + 8) * 4;
-    return (size_t)n * per + hist + 256 * (15 + Q_COUNT + 6) + C_WORDS * kCtrStride * 4 + 4096;
+    return (size_t)n * per + hist + 256 * (17 + Q_COUNT + 6) + C_WORDS * kCtrStride * 4 + 4096;
 }
 
 void WavefrontStateFree(WavefrontState* wf) {
@@ -1076,7 +1106,7 @@ int WavefrontPass(Ctx* c, Scene* sc, const PathParams& P, const gy_render_params
     Rd.F = FilmView(sc);
     hipLaunchKernelGGL(k_wf_reset, dim3(1), dim3(64), 0, c->stream, W);
     TimerBegin(c, kKernRaygen);
-    hipLaunchKernelGGL(k_wf_raygen, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, c->stream, W, P, s0, n_s, width, height);
+    hipLaunchKernelGGL(k_wf_raygen, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, c->stream, W, P, Rd.F, s0, n_s);
     TimerEnd(c);
     rc = CheckLaunch(c, "k_wf_raygen");
     if (rc != GY_OK) return rc;
@@ -1098,7 +1128,7 @@ int WavefrontPass(Ctx* c, Scene* sc, const PathParams& P, const gy_render_params
 // (k_wf_trace MODE 0), makes each hit a vertex (k_lt_shade: its camera
 // connection and its next ray), then traces the connections (MODE 3, the
 // shadow queue), which splats the unoccluded ones as they finish.  Per lane:
-// o, d the extension ray, T the throughput, seq (index, cursor, bounce),
+// o, d the extension ray, T the throughput and state (cursor, bounce), idx the index,
 // sh_o / sh_d the connection ray (tmax in sh_o.w), pend0 its splat (L, pixel).
 struct LtArgs {
     LightCamDev C;
@@ -1139,7 +1169,7 @@ __device__ inline bool lt_prepare(const WfDev& W, const LtArgs& A, uint32_t slot
     int Y = iy < 0 ? 0 : (iy > C.height - 1 ? C.height - 1 : iy);
     const V3 so = pos + toCam * kRayEps;
     W.sh_o[slot] = make_float4(so.x, so.y, so.z, len);
-    W.sh_d[slot] = make_float4(toCam.x, toCam.y, toCam.z, 0.f);
+    W.sh_d[slot] = toCam;
     W.pend0[slot] = make_float4(L.x, L.y, L.z, __uint_as_float((uint32_t)(Y * C.width + X)));
     return true;
 }
@@ -1174,10 +1204,10 @@ __global__ void __launch_bounds__(256) k_lt_start(SceneDev S, PathParams P, WfDe
         }
         const V3 T = Le * fabsf(dot(ln, dir)) / pdfLight / pdfA / pdfDir;
         const V3 o = (lpos + dir * kRayEps) + dir * kRayEps;
-        W.o[slot] = make_float4(o.x, o.y, o.z, 0.f);
-        W.d[slot] = make_float4(dir.x, dir.y, dir.z, 0.f);
-        W.T[slot] = make_float4(T.x, T.y, T.z, 0.f);
-        W.seq[slot] = make_uint4((uint32_t)q.index, (uint32_t)(q.index >> 32), q.cursor, 1u);
+        W.o[slot] = o;
+        W.d[slot] = dir;
+        W.T[slot] = make_float4(T.x, T.y, T.z, __uint_as_float(st_pack(q.cursor, 1u, false, 0u)));
+        W.idx[slot] = make_uint2((uint32_t)q.index, (uint32_t)(q.index >> 32));
     }
     uint32_t* const qs[2] = {W.q[Q_SHADOW], W.q[Q_NEXT]};
     uint32_t* const cs[2] = {&W.counts[Q_SHADOW * kCtrStride], &W.counts[Q_NEXT * kCtrStride]};
@@ -1195,24 +1225,26 @@ __global__ void __launch_bounds__(256) k_lt_shade(SceneDev S, PathParams P, WfDe
     bool conn = false, next = false;
     if (i < n && W.mtype[W.q[Q_ACTIVE][i]] != 255) {
         slot = W.q[Q_ACTIVE][i];
-        const V3 o = f3(W.o[slot]), d = f3(W.d[slot]);
-        const float4 hv = W.hit[slot];
+        const V3 o = W.o[slot], d = W.d[slot];
+        const HitRec hv = W.hit[slot];
         Hit h;
-        h.t = hv.x;
-        h.prim = __float_as_int(hv.y);
-        h.b1 = hv.z;
-        h.b2 = hv.w;
+        h.t = 0.f;  // not read
+        h.prim = hv.prim;
+        h.b1 = hv.b1;
+        h.b2 = hv.b2;
         const Isect it = query(S, o, d, h);
         BSDF b = make_bsdf(S, it);
         b.importance = true;  // ComputeScatteringFunction(arena, TransportMode::Importance) (integrator/LT.h:69)
-        V3 T = f3(W.T[slot]);
+        const float4 Tv = W.T[slot];
+        const uint32_t st = __float_as_uint(Tv.w);
+        V3 T = f3(Tv);
         conn = lt_prepare(W, A, slot, it.pos, it.n, it.outDir, &b, T, false);
-        uint4 sq = W.seq[slot];
-        const uint32_t bounce = sq.w + 1u;
+        const uint32_t bounce = ((st >> kStDepth) & kStDepthMask) + 1u;
         if ((int)bounce < A.max_depth) {
             Seq q;
-            q.index = (uint64_t)sq.x | ((uint64_t)sq.y << 32);
-            q.cursor = sq.z;
+            const uint2 ix = W.idx[slot];
+            q.index = (uint64_t)ix.x | ((uint64_t)ix.y << 32);
+            q.cursor = st & kStCursor;
             const SampleSrc& M = P.smp;
             const float r0 = seq_next_wide(M, q), r1 = seq_next_wide(M, q), r2 = seq_next_wide(M, q);
             V3 wi;
@@ -1220,10 +1252,9 @@ __global__ void __launch_bounds__(256) k_lt_shade(SceneDev S, PathParams P, WfDe
             const V3 f = bsdf_sample(b, neg(d), &wi, &pdfDir, r0, r1, r2);
             const V3 no = (it.pos + wi * kRayEps) + wi * kRayEps;
             T = T * f * fabsf(dot(wi, it.n)) / pdfDir;
-            W.o[slot] = make_float4(no.x, no.y, no.z, 0.f);
-            W.d[slot] = make_float4(wi.x, wi.y, wi.z, 0.f);
-            W.T[slot] = make_float4(T.x, T.y, T.z, 0.f);
-            W.seq[slot] = make_uint4(sq.x, sq.y, q.cursor, bounce);
+            W.o[slot] = no;
+            W.d[slot] = wi;
+            W.T[slot] = make_float4(T.x, T.y, T.z, __uint_as_float(st_pack(q.cursor, bounce, false, 0u)));
             next = true;
         }
     }
