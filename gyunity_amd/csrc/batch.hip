@@ -30,7 +30,7 @@ int BatchBuild(Ctx* c, Batch* b, int64_t lanes_req) {
     if (b->entries.empty()) return Fail(GY_ERR_INVALID, "gy_batch_render: empty batch");
     BatchDropGraph(b);
     std::vector<BatchEntryDev> tab(b->entries.size());
-    int64_t first = 0, image_off = 0, adj_blocks = 0;
+    int64_t first = 0, first_valid = 0, image_off = 0, adj_blocks = 0;
     int depth_max = 0;
     b->rendered = false;
     for (size_t i = 0; i < b->entries.size(); ++i) {
@@ -50,12 +50,15 @@ int BatchBuild(Ctx* c, Batch* b, int64_t lanes_req) {
         d.tilesY = (H + 7) >> 3;
         d.paths = (int64_t)d.tilesX * d.tilesY * 64 * en.params.spp;
         d.first = first;
+        d.first_valid = first_valid;
         d.image_off = image_off;
         d.adj_block0 = adj_blocks;
         en.first = first;
+        en.first_valid = first_valid;
         en.paths = d.paths;
         en.image_off = image_off;
         first += d.paths;
+        first_valid += (int64_t)W * H * en.params.spp;
         image_off += (int64_t)W * H * 3;
         adj_blocks += (d.paths + kBatchAdjointBlock - 1) / kBatchAdjointBlock;
         depth_max = std::max(depth_max, en.params.max_depth);

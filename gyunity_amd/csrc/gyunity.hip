@@ -499,6 +499,7 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     sc->area_le.assign(d.light_le, d.light_le + 3 * (size_t)nl);
     std::vector<float> func = sc->area_func, cdf;
     const float func_int = LightCdf(func, &cdf);
+    for (int i = 0; i < d.n_mat; ++i) sc->mat_types |= 1u << d.mats[(size_t)i * GY_MAT_WORDS];
     sc->dev.light_func_int = func_int;
     sc->dev.n_light = nl;
     sc->dev.n_tri = d.n_tri;

@@ -77,6 +77,7 @@ struct WavefrontState {
 struct Scene {
     Ctx* ctx = nullptr;
     int32_t n_tri = 0;
+    uint32_t mat_types = 0;  // one bit per material type (GY_MAT_*) the scene holds
     int32_t batch_refs = 0;  // batch entries that render this scene
     gyd::SceneDev dev = {};
     void *d_tri = nullptr, *d_shade = nullptr, *d_nodes = nullptr, *d_mats = nullptr, *d_tex = nullptr, *d_texinfo = nullptr;
@@ -146,6 +147,7 @@ struct BatchEntryDev {
     PathParams P;
     FilmDev F;
     int64_t first;  // first global path index of the entry
+    int64_t first_valid;  // paths with a pixel in the entries before
     int64_t paths;  // tile-padded paths: tilesX * tilesY * 64 * spp
     int64_t image_off;  // the entry's first float in the batch's concatenated images (W * H * 3 per entry)
     int64_t adj_block0; // the entry's first workgroup in the batch adjoint launch (kBatchAdjointBlock lanes each)
@@ -158,7 +160,7 @@ struct BatchEntry {
     gy_render_params params = {};
     PathParams P = {};
     FilmState film;
-    int64_t first = 0, paths = 0;
+    int64_t first = 0, first_valid = 0, paths = 0;
     int64_t image_off = 0;
     uint64_t tex_revision = 0;  // the scene's texture revision the last batch render saw
     uint64_t scene_revision = 0;  // the scene's revision when the table was built

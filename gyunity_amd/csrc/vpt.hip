@@ -498,7 +498,12 @@ __global__ void __launch_bounds__(128) k_vpt_li_samples(SceneDev S, MediaDev M, 
 enum VwfQueue { VQ_ACTIVE = 0, VQ_NEXT = 1, VQ_SHADOW = 2, VQ_MIS = 3, VQ_COUNT = 4 };
 constexpr int kVwfCtr = 32;                  // counter stride in words (one 128-byte line each)
 constexpr int kVwfChunks = 8;                // queue chunks a trace launch claims from, one per XCD
-constexpr int kVwfWords = VQ_COUNT + 3 * kVwfChunks;  // queue lengths, then the fetch counters of each trace mode
+// The shadow and MIS queues have a part with its own length per chunk, and a
+// vertex workgroup pushes to part blockIdx % 8: same-address atomics take 11 ns
+// each, one per workgroup and queue.
+constexpr int kVwfPart0 = VQ_COUNT + 3 * kVwfChunks;
+constexpr int kVwfWords = kVwfPart0 + 2 * kVwfChunks;  // queue lengths, the fetch counters of each trace mode, part lengths
+static_assert(kVwfWords <= 64, "one wave advances them");
 // Path flags (pk): the slot holds a path; its vertex set up direct light (DI)
 // or an equi-angular connection (CONN, CONN0 when the light faces away); a
 // shadow or MIS segment was traced for it; the path ends after this round.
@@ -525,6 +530,7 @@ struct VwfDev {
     uint32_t* q[VQ_COUNT];
     uint32_t* counts;
     int64_t capacity;
+    uint32_t part;  // room in each part of the shadow and MIS queues
     uint32_t* spill;
     int64_t spill_stride;
 };
@@ -846,8 +852,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
         }
         W.pk[slot] = pk | (ends ? VK_DONE : 0u);
     }
-    uint32_t* const qs[2] = {W.q[VQ_SHADOW], W.q[VQ_MIS]};
-    uint32_t* const cs[2] = {&W.counts[VQ_SHADOW * kVwfCtr], &W.counts[VQ_MIS * kVwfCtr]};
+    const uint32_t c = blockIdx.x % kVwfChunks;
+    uint32_t* const qs[2] = {W.q[VQ_SHADOW] + (size_t)c * W.part, W.q[VQ_MIS] + (size_t)c * W.part};
+    uint32_t* const cs[2] = {&W.counts[(kVwfPart0 + c) * kVwfCtr], &W.counts[(kVwfPart0 + kVwfChunks + c) * kVwfCtr]};
     const uint32_t it[1] = {slot};
     const bool pr[2][1] = {{push_sh}, {push_mis}};
     vwf_block_push<2, 1>(qs, cs, it, pr);
@@ -865,8 +872,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 template <int S, int MODE, bool ENV>
 __device__ inline void vwf_trace_loop(const SceneDev& Sc, const MediaDev& M, const VwfDev& W, int refill, uint32_t* stack) {
     constexpr int qid = MODE == 0 ? VQ_ACTIVE : (MODE == 1 ? VQ_SHADOW : VQ_MIS);
-    const uint32_t n = W.counts[qid * kVwfCtr];
-    // The queue is cut into kVwfChunks regions with a fetch counter each; a
+    const uint32_t n = MODE == 0 ? W.counts[qid * kVwfCtr] : 0u;
+    // The active queue is cut into kVwfChunks regions with a fetch counter each; a
     // wave starts on the region of its XCD (workgroups are dealt to the XCDs
     // round-robin) and moves on when it runs dry, so no one counter takes
     // every claim.
@@ -891,10 +898,20 @@ __device__ inline void vwf_trace_loop(const SceneDev& Sc, const MediaDev& M, con
         while (nm) {
             if (batch_left == 0) {
                 while (tries < kVwfChunks) {
-                    const uint32_t lo = (uint32_t)(((uint64_t)n * ck) / kVwfChunks);
-                    const uint32_t hi = (uint32_t)(((uint64_t)n * (ck + 1)) / kVwfChunks);
-                    uint32_t base = 0;
-                    if (lane == 0) base = atomicAdd(&fetch[ck * kVwfCtr], 64u);
+                    uint32_t lo, hi;
+                    if (MODE == 0) {
+                        lo = (uint32_t)(((uint64_t)n * ck) / kVwfChunks);
+                        hi = (uint32_t)(((uint64_t)n * (ck + 1)) / kVwfChunks);
+                    } else {
+                        lo = (uint32_t)ck * W.part;
+                        hi = lo + W.counts[(kVwfPart0 + (MODE - 1) * kVwfChunks + ck) * kVwfCtr];
+                    }
+                    // a chunk that is not the wave's own is looked at before it is
+                    // claimed from (a same-address atomic takes 11 ns, and at the
+                    // end of a launch every wave looks at every chunk)
+                    uint32_t base = hi - lo;
+                    if (lane == 0 && (tries == 0 || __hip_atomic_load(&fetch[ck * kVwfCtr], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < hi - lo))
+                        base = atomicAdd(&fetch[ck * kVwfCtr], 64u);
                     base = __shfl(base, 0, 64);
                     if (base < hi - lo) {
                         batch_base = lo + base;
@@ -1094,16 +1111,16 @@ __global__ void __launch_bounds__(256) k_vwf_resolve(VwfDev W, FilmDev F, int64_
 }
 
 // Next round: the next queue becomes the active one; returns its length.
-__global__ void k_vwf_advance(VwfDev W, uint32_t* out, unsigned long long* rays) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        rays[0] += W.counts[VQ_ACTIVE * kVwfCtr];
-        rays[1] += W.counts[VQ_SHADOW * kVwfCtr];
-        rays[2] += W.counts[VQ_MIS * kVwfCtr];
-        const uint32_t nx = W.counts[VQ_NEXT * kVwfCtr];
-        for (int w = 0; w < kVwfWords; ++w) W.counts[w * kVwfCtr] = 0u;
-        W.counts[VQ_ACTIVE * kVwfCtr] = nx;
+__global__ void k_vwf_advance(VwfDev W, uint32_t* out, unsigned long long* rays) {  // one wave
+    const int w = threadIdx.x;
+    const uint32_t v = w < kVwfWords ? W.counts[w * kVwfCtr] : 0u;
+    const uint32_t nx = __shfl(v, VQ_NEXT, 64);
+    if (w == VQ_ACTIVE) {
+        rays[0] += v;
         *out = nx;
     }
+    if (w >= kVwfPart0 && w < kVwfWords && v) atomicAdd(&rays[w < kVwfPart0 + kVwfChunks ? 1 : 2], (unsigned long long)v);
+    if (w < kVwfWords) W.counts[w * kVwfCtr] = w == VQ_ACTIVE ? nx : 0u;
 }
 __global__ void k_vwf_reset(VwfDev W) {
     if (threadIdx.x < kVwfWords && blockIdx.x == 0) W.counts[threadIdx.x * kVwfCtr] = 0u;
@@ -1146,9 +1163,11 @@ int LaunchVpt(Ctx* c, Scene* sc, const PathParams& P, int s0, int n_s, bool eqa)
 constexpr int kVwfStack = 16;  // LDS stack entries per lane; deeper ones spill
 constexpr int kVwfRefill = 48;
 
+// One part takes the pushes of one workgroup in eight of a vertex launch.
+static uint32_t VwfPartRoom(int64_t n) { return (uint32_t)(((n + kVwfChunks - 1) / kVwfChunks + 2 * 256 + 255) / 256 * 256); }
 static size_t VwfBytes(int64_t n) {
     const size_t per = 24 * 16 + 4 + 4 + VQ_COUNT * 4;  // 24 float4 / uint4 arrays, med, pk, queues
-    return (size_t)n * per + 256 * (24 + 2 + VQ_COUNT + 2) + kVwfWords * kVwfCtr * 4 + 4096;
+    return (size_t)n * per + 2 * ((size_t)VwfPartRoom(n) * kVwfChunks - n) * 4 + 256 * (24 + 2 + VQ_COUNT + 2) + kVwfWords * kVwfCtr * 4 + 4096;
 }
 static VwfDev VwfView(const WavefrontState& wf, size_t* used) {
     VwfDev W;
@@ -1166,7 +1185,9 @@ static VwfDev VwfView(const WavefrontState& wf, size_t* used) {
     W.st = (uint4*)take(n * 16);
     W.med = (int32_t*)take(n * 4);
     W.pk = (uint32_t*)take(n * 4);
-    for (int q = 0; q < VQ_COUNT; ++q) W.q[q] = (uint32_t*)take(n * 4);
+    W.part = VwfPartRoom(n);
+    for (int q = 0; q < VQ_COUNT; ++q)
+        W.q[q] = (uint32_t*)take(q == VQ_SHADOW || q == VQ_MIS ? (size_t)W.part * kVwfChunks * 4 : (size_t)n * 4);
     W.counts = (uint32_t*)take((size_t)(kVwfWords + 1) * kVwfCtr * 4);  // + the round's active count for the host
     W.capacity = n;
     W.spill = (uint32_t*)wf.spill;

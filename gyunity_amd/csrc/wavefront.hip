@@ -40,7 +40,10 @@ enum QueueId { Q_ACTIVE = 0, Q_NEXT = 1, Q_SHADE0 = 2, Q_SHADOW = 6, Q_MIS = 7, 
 // eight per trace MODE 0..3 (one per queue chunk, see k_wf_trace)
 constexpr int C_FETCH0 = 16;
 constexpr int kChunks = 8;  // XCDs of the device; workgroup b runs on XCD b % 8
-constexpr int C_WORDS = 48;
+// words 48..63: lengths of the eight parts of the shadow and the MIS queue
+constexpr int kParts = 8;
+constexpr int C_PART0 = 48;
+constexpr int C_WORDS = 64;
 // Each counter sits in its own 128-byte line, so that atomics on different
 // queues do not serialise on one L2 channel.
 constexpr int kCtrStride = 32;
@@ -107,7 +110,8 @@ struct WfDev {
     const uint32_t* trace_q;  // queue of the closest-hit trace when it differs from the active queue (else null)
     uint32_t* sort_hist;   // ray sort: 8 x sort_blocks octant counts, then their offsets; 8 octant totals
     uint32_t sort_blocks;  // ray sort: workgroups of kSortPer queue entries over the capacity
-    uint32_t* counts;          // Q_COUNT counters
+    uint32_t* counts;          // C_WORDS counters
+    uint32_t part;             // room in each part of the shadow and MIS queues
     int64_t capacity;
     uint32_t* spill;       // traversal stack entries beyond the LDS part, entry-major
     int64_t spill_stride;  // lanes per launch (grid size)
@@ -173,6 +177,19 @@ __device__ inline void block_push(uint32_t* const (&q)[NQ], uint32_t* const (&cn
     }
 }
 
+// Shading's shadow and MIS pushes.  Same-address atomics serialise (about 11 ns
+// each, which bounded shading: 170,000 workgroups of a 43M-point launch are
+// 1.9 ms of one counter), so each of the two queues has eight parts with a
+// counter each, and workgroup b pushes to part b % 8: the part that the trace
+// waves of its XCD start on.
+__device__ inline void part_push(const WfDev& W, uint32_t slot, bool shadow, bool mis) {
+    const uint32_t c = blockIdx.x % kParts;
+    uint32_t* const q[2] = {W.q[Q_SHADOW] + (size_t)c * W.part, W.q[Q_MIS] + (size_t)c * W.part};
+    uint32_t* const n[2] = {&W.counts[(C_PART0 + c) * kCtrStride], &W.counts[(C_PART0 + kParts + c) * kCtrStride]};
+    const bool p[2] = {shadow, mis};
+    block_push<2>(q, n, slot, p);
+}
+
 // One queue, K items per thread, one atomic per workgroup.  Item k of thread t
 // ranks at (k, t): entries keep the order of k * 256 + t.
 template <int K>
@@ -225,7 +242,24 @@ __device__ inline void start_path(const WfDev& W, const PathParams& P, const Fil
     W.flags[slot] = P.max_depth == 0 ? P_DONE : 0u;
 }
 
+// Lanes before lane r of one sample's 8x8-tile order that have a pixel.
+__host__ __device__ inline int64_t tile_rank(int width, int height, int64_t r) {
+    const int tilesX = (width + 7) >> 3;
+    const int64_t tile = r >> 6;
+    const int local = (int)(r & 63), x0 = (int)(tile % tilesX) * 8;
+    const int64_t y0 = tile / tilesX * 8;
+    if (y0 >= height) return (int64_t)width * height;
+    const int h = height - y0 < 8 ? (int)(height - y0) : 8, w = width - x0 < 8 ? width - x0 : 8;
+    const int ly = local >> 3, lx = local & 7;
+    const int in_tile = ly < h ? ly * w + (lx < w ? lx : w) : h * w;
+    return y0 * width + (int64_t)x0 * h + in_tile;
+}
+
 // ---------------------------------------------------------------- raygen
+// A path's place in the first active queue follows from its pixel alone (the
+// lanes of a ragged image's last tiles that have none are skipped), so raygen
+// claims nothing: with an atomic per workgroup it took 3.0 ms for 67M paths, the
+// 262,144 atomics' time.
 // One render: samples s0 .. s0+n_s-1 of every pixel, 8x8 pixel tiles per wave.
 __global__ void __launch_bounds__(256) k_wf_raygen(WfDev W, PathParams P, FilmDev F, int s0, int n_s) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -244,17 +278,20 @@ __global__ void __launch_bounds__(256) k_wf_raygen(WfDev W, PathParams P, FilmDe
         valid = px < width && py < height;
     }
     const uint32_t slot = (uint32_t)((int64_t)s_local * width * height + (int64_t)py * width + px);
-    if (valid) start_path(W, P, F, slot, s0 + s_local, px, py);
-    uint32_t* const qa[1] = {W.q[Q_ACTIVE]};
-    uint32_t* const ca[1] = {&W.counts[Q_ACTIVE * kCtrStride]};
-    const bool pa[1] = {valid};
-    block_push<1>(qa, ca, slot, pa);
+    if (valid) {
+        start_path(W, P, F, slot, s0 + s_local, px, py);
+        const int64_t r = t - (int64_t)s_local * per_s;
+        W.q[Q_ACTIVE][(int64_t)s_local * width * height + tile_rank(width, height, r)] = slot;
+    }
+    if (t == 0) W.counts[Q_ACTIVE * kCtrStride] = (uint32_t)((int64_t)width * height * n_s);
 }
 
+// valid0: paths with a pixel before `base`; n_valid: among these lanes.
 // Batch: lanes [0, count) take global path indices base + lane.  Entry e owns
 // global indices [E[e].first, E[e].first + E[e].paths) in its own tile order
 // (sample-major, 8x8 pixel tiles); the lane records its entry and pass slot.
-__global__ void __launch_bounds__(256) k_wf_raygen_batch(WfDev W, ManyRenders R, int64_t base, int64_t count, int64_t lanes) {
+__global__ void __launch_bounds__(256) k_wf_raygen_batch(WfDev W, ManyRenders R, int64_t base, int64_t count, int64_t lanes,
+                                                         int64_t valid0, uint32_t n_valid) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     bool valid = t < count;
     uint32_t e = 0;
@@ -282,16 +319,17 @@ __global__ void __launch_bounds__(256) k_wf_raygen_batch(WfDev W, ManyRenders R,
     const uint32_t slot = (uint32_t)t;
     if (valid) {
         const PathParams& P = R.E[e].P;
+        const BatchEntryDev& B = R.E[e];
+        const int64_t r = base + t - B.first, per_s = (int64_t)B.tilesX * B.tilesY * 64;
+        W.q[Q_ACTIVE][B.first_valid - valid0 + (int64_t)s * P.cam.width * P.cam.height +
+                      tile_rank(P.cam.width, P.cam.height, r - (int64_t)s * per_s)] = slot;
         W.ent[slot] = e;
         W.pslot[slot] = (uint32_t)((int64_t)s * P.cam.width * P.cam.height + (int64_t)py * P.cam.width + px);
         start_path(W, P, R.E[e].F, slot, s, px, py);
     } else if (t < lanes) {
         W.flags[slot] = 0u;  // resolve walks every lane: one without a path has no flags
     }
-    uint32_t* const qa[1] = {W.q[Q_ACTIVE]};
-    uint32_t* const ca[1] = {&W.counts[Q_ACTIVE * kCtrStride]};
-    const bool pa[1] = {valid};
-    block_push<1>(qa, ca, slot, pa);
+    if (t == 0) W.counts[Q_ACTIVE * kCtrStride] = n_valid;
 }
 
 // ---------------------------------------------------------------- persistent trace
@@ -304,16 +342,24 @@ __global__ void __launch_bounds__(256) k_wf_raygen_batch(WfDev W, ManyRenders R,
 // idle lanes then take new entries.  A wave exits when the queue is drained
 // and none of its lanes holds a ray.
 constexpr uint32_t kBatch = 64;
+// Whether a chunk's fetch counter is below its length.  A wave asks before it
+// claims from a chunk that is not its own: at the end of a launch every resident
+// wave (6144) looks at all eight chunks, and with an atomic for each look the
+// counters alone took 67 us of every trace loop (11 ns a same-address atomic).
+__device__ inline bool fetch_left(const uint32_t* fetch, uint32_t len) {
+    return __hip_atomic_load(fetch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < len;
+}
 
 template <int S, int MODE, class R>
 __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, int chunks, uint32_t* stack) {
     constexpr bool kAny = MODE == 1 || MODE == 3;
     constexpr int qid = MODE == 0 ? Q_ACTIVE : (kAny ? Q_SHADOW : Q_MIS);
-    const uint32_t n = W.counts[(qid) * kCtrStride];
-    // The queue is cut into kChunks contiguous chunks, one per XCD.  Workgroups
-    // are dealt to the XCDs round-robin, so a wave starts on its own XCD's
-    // chunk, where its rays are neighbours of the rays the XCD's L2 already
-    // holds nodes for, and steals from the next chunks once that one is empty.
+    const uint32_t n = MODE == 0 ? W.counts[(qid) * kCtrStride] : 0u;
+    // The closest-hit queue is cut into contiguous chunks, one per XCD; the
+    // others have their parts (part_push).  Workgroups are dealt to the XCDs
+    // round-robin, so a wave starts on its own XCD's chunk, where its rays are
+    // neighbours of the rays the XCD's L2 already holds nodes for, and steals
+    // from the next chunks once that one is empty.
     uint32_t* fetch = &W.counts[(C_FETCH0 + MODE * kChunks) * kCtrStride];
     int ck = (int)(blockIdx.x % kChunks) % chunks, tries = 0;  // wave-uniform
     const int lane = threadIdx.x & 63;
@@ -335,10 +381,17 @@ __device__ inline void wf_trace_loop(const R& Rd, const WfDev& W, int refill, in
         while (nm) {
             if (batch_left == 0) {
                 while (tries < chunks) {
-                    const uint32_t lo = (uint32_t)(((uint64_t)n * ck) / chunks);
-                    const uint32_t hi = (uint32_t)(((uint64_t)n * (ck + 1)) / chunks);
-                    uint32_t base = 0;
-                    if (lane == 0) base = atomicAdd(&fetch[ck * kCtrStride], (uint32_t)kBatch);
+                    uint32_t lo, hi;
+                    if (MODE == 0) {
+                        lo = (uint32_t)(((uint64_t)n * ck) / chunks);
+                        hi = (uint32_t)(((uint64_t)n * (ck + 1)) / chunks);
+                    } else {
+                        lo = (uint32_t)ck * W.part;
+                        hi = lo + W.counts[(C_PART0 + (kAny ? 0 : kParts) + ck) * kCtrStride];
+                    }
+                    uint32_t base = hi - lo;
+                    if (lane == 0 && (tries == 0 || fetch_left(&fetch[ck * kCtrStride], hi - lo)))
+                        base = atomicAdd(&fetch[ck * kCtrStride], (uint32_t)kBatch);
                     base = __shfl(base, 0, 64);
                     if (base < hi - lo) {
                         batch_base = lo + base;
@@ -607,9 +660,11 @@ __global__ void __launch_bounds__(256) k_wf_sort_scatter(WfDev W) {
 // this pass bins the active queue into the four shade queues in queue order.
 // The order of the shade queues (neighbouring paths together) then does not
 // depend on when each ray finished, which lets the
-// closest-hit waves refill early.  Each thread takes four consecutive entries
-// and the workgroup claims its block of each queue with one atomic.
-constexpr int kBinPerThread = 4;
+// closest-hit waves refill early.  Each thread takes sixteen consecutive
+// entries and the workgroup claims its block of each queue with one atomic (with
+// four entries a thread the atomics, 11 ns each, were most of its 0.46 ms a
+// bounce of 67M paths).
+constexpr int kBinPerThread = 16;
 __global__ void __launch_bounds__(256) k_wf_bin(WfDev W) {
     __shared__ uint64_t wsum[4];
     __shared__ uint32_t base[4];
@@ -665,9 +720,13 @@ __global__ void __launch_bounds__(256) k_wf_bin(WfDev W) {
 // stored as L2 w2 like a hit of an area light.
 template <int MODE, class R>
 __global__ void __launch_bounds__(256) k_wf_env(R Rd, WfDev W) {
-    const uint32_t n = W.counts[(MODE == 0 ? Q_ACTIVE : Q_MIS) * kCtrStride];
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
+    if (MODE == 0) {
+        if (i >= W.counts[Q_ACTIVE * kCtrStride]) return;
+    } else {
+        const uint32_t c = i / W.part;
+        if (c >= (uint32_t)kParts || i - c * W.part >= W.counts[(C_PART0 + kParts + c) * kCtrStride]) return;
+    }
     const uint32_t slot = W.q[MODE == 0 ? Q_ACTIVE : Q_MIS][i];
     const SceneDev& S = Rd.scene(Rd.entry(W, slot));
     if (S.env.w == 0) return;
@@ -842,10 +901,7 @@ __global__ void __launch_bounds__(256) k_wf_shade(R Rd, WfDev W) {
         if (alive) W.T[slot] = make_float4(T.x, T.y, T.z, __uint_as_float(nst));
         W.flags[slot] = alive ? (pflags ? pflags : P_NEXT) : (pflags | P_DONE);
     }
-    uint32_t* const qs[2] = {W.q[Q_SHADOW], W.q[Q_MIS]};
-    uint32_t* const cs[2] = {&W.counts[Q_SHADOW * kCtrStride], &W.counts[Q_MIS * kCtrStride]};
-    const bool ps[2] = {push_shadow, push_mis};
-    block_push<2>(qs, cs, slot, ps);
+    part_push(W, slot, push_shadow, push_mis);
 }
 
 // ---------------------------------------------------------------- resolve
@@ -892,36 +948,51 @@ __device__ inline bool resolve_slot(const R& Rd, const WfDev& W, uint32_t slot) 
 // path records of neighbouring slots together.  A slot with no flags costs one
 // 4-byte load.  A path that goes on keeps its flags, which the next bounce
 // rewrites (shading, or the closest-hit miss) before they are read again.
-constexpr int kResolvePerThread = 4;
+// Sixteen slots a thread, four at a time: one atomic per 4096 slots (at 1024
+// the atomics alone, 11 ns each, took 0.7 ms of a 67M-slot launch).
+constexpr int kResolvePerThread = 16;
 template <class R>
 __global__ void __launch_bounds__(256) k_wf_resolve(R Rd, WfDev W, uint32_t n) {
+    const uint32_t base = blockIdx.x * kResolvePerThread * 256 + threadIdx.x;
+    uint32_t goes_on = 0;  // one bit per slot
+    for (int g = 0; g < kResolvePerThread; g += 4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t slot = base + (g + k) * 256;
+            if (slot < n && resolve_slot(Rd, W, slot)) goes_on |= 1u << (g + k);
+        }
+    }
     uint32_t slot[kResolvePerThread];
     bool next[kResolvePerThread];
 #pragma unroll
     for (int k = 0; k < kResolvePerThread; ++k) {
-        slot[k] = (blockIdx.x * kResolvePerThread + k) * 256 + threadIdx.x;
-        next[k] = slot[k] < n && resolve_slot(Rd, W, slot[k]);
+        slot[k] = base + k * 256;
+        next[k] = (goes_on >> k) & 1u;
     }
     block_push_items<kResolvePerThread>(W.q[Q_NEXT], &W.counts[Q_NEXT * kCtrStride], slot, next);
 }
 
 // Queue bookkeeping between bounces: next -> active, counters reset.
-__global__ void k_wf_advance(WfDev W, unsigned long long* ctr) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        // rays traced this bounce: camera/continuation, shadow, MIS
-        ctr[0] += W.counts[(Q_ACTIVE) * kCtrStride];
-        ctr[1] += W.counts[(Q_SHADOW) * kCtrStride];
-        ctr[2] += W.counts[(Q_MIS) * kCtrStride];
-        W.counts[(Q_ACTIVE) * kCtrStride] = W.counts[(Q_NEXT) * kCtrStride];
-        W.counts[(Q_NEXT) * kCtrStride] = 0;
-        for (int q = Q_SHADE0; q < C_WORDS; ++q) W.counts[(q) * kCtrStride] = 0;
-    }
+__global__ void k_wf_advance(WfDev W, unsigned long long* ctr) {  // one wave
+    const int w = threadIdx.x;
+    uint32_t v = W.counts[w * kCtrStride];
+    // rays traced this bounce: camera/continuation, shadow, MIS
+    uint32_t part = v;
+    for (int d = 1; d < kParts; d <<= 1) part += __shfl_xor(part, d, 64);
+    if (w == Q_ACTIVE) ctr[0] += v;
+    if (w == C_PART0) ctr[1] += part;
+    if (w == C_PART0 + kParts) ctr[2] += part;
+    const uint32_t next = __shfl(v, Q_NEXT, 64);
+    W.counts[w * kCtrStride] = w == Q_ACTIVE ? next : 0u;
 }
 __global__ void k_wf_reset(WfDev W) {
     if (threadIdx.x < C_WORDS && blockIdx.x == 0) W.counts[(threadIdx.x) * kCtrStride] = 0;
 }
 
 // ---------------------------------------------------------------- host side
+// Room in one part of the shadow and MIS queues: at most one workgroup in eight
+// of each of the four shading launches pushes to it, 256 entries each.
+static uint32_t PartRoom(int64_t n) { return (uint32_t)(((n + kParts - 1) / kParts + 4 * 2 * 256 + 255) / 256 * 256); }
 static WfDev g_view(const WavefrontState& wf, bool batch, size_t* used) {
     WfDev W;
     char* base = (char*)wf.mem;
@@ -951,7 +1022,9 @@ static WfDev g_view(const WavefrontState& wf, bool batch, size_t* used) {
     W.mis_d = (V3*)take(n * 12);
     W.ent = batch ? (uint32_t*)take(n * 4) : nullptr;
     W.pslot = batch ? (uint32_t*)take(n * 4) : nullptr;
-    for (int q = 0; q < Q_COUNT; ++q) W.q[q] = (uint32_t*)take(n * 4);
+    W.part = PartRoom(n);
+    for (int q = 0; q < Q_COUNT; ++q)
+        W.q[q] = (uint32_t*)take(q == Q_SHADOW || q == Q_MIS ? (size_t)W.part * kParts * 4 : (size_t)n * 4);
     W.sort_blocks = (uint32_t)((n + kSortPer - 1) / kSortPer);
     W.sort_q = (uint32_t*)take(n * 4);
     W.trace_q = nullptr;
@@ -967,7 +1040,7 @@ static WfDev g_view(const WavefrontState& wf, bool batch, size_t* used) {
 static size_t WfBytes(int64_t n, bool batch) {
     const size_t per = 5 * 16 + 9 * 12 + 8 + 4 + 1 + (Q_COUNT + 1) * 4 + (batch ? 8 : 0);
     const size_t hist = ((size_t)((n + kSortPer - 1) / kSortPer) * 8 + 8) * 4;
-    return (size_t)n * per + hist + 256 * (17 + Q_COUNT + 6) + C_WORDS * kCtrStride * 4 + 4096;
+    return (size_t)n * per + 2 * ((size_t)PartRoom(n) * kParts - n) * 4 + hist + 256 * (17 + Q_COUNT + 6) + C_WORDS * kCtrStride * 4 + 4096;
 }
 
 void WavefrontStateFree(WavefrontState* wf) {
@@ -1019,16 +1092,16 @@ static int WfPrepareState(Ctx* c, WavefrontState& wf, int64_t n, bool batch, int
 // active / next queue pointers swap on the host between bounces, fixed per
 // launch, so the whole sequence can be recorded in a graph.
 // Launch shape of the three trace kinds.  Queue chunks: closest-hit rays are
-// claimed from eight regions of the queue at once (one per XCD), shadow rays
-// from four, MIS rays from one.  Automatic refill: a lane takes a new ray once
+// claimed from eight regions of the queue at once (one per XCD), shadow and MIS
+// rays from their eight parts.  Automatic refill: a lane takes a new ray once
 // fewer than 48 lanes of its wave are still traversing.  Refilling does not
 // reorder the shade queues, which k_wf_bin builds in queue order.
 static unsigned ResolveBlocks(uint32_t n) { return (unsigned)(((uint64_t)n + 256 * kResolvePerThread - 1) / (256 * kResolvePerThread)); }
-constexpr int kTraceChunks[3] = {8, 4, 1};
+constexpr int kTraceChunks[3] = {8, kParts, kParts};
 constexpr int kAutoRefill = 48;
 template <int STACK, class R>
 static int WfBounceLoop(Ctx* c, const R& Rd, const WfDev& W0, int depth_max, int refill, int ray_sort, unsigned blocks,
-                        uint32_t n_slots, bool env, unsigned long long* counters) {
+                        uint32_t n_slots, bool env, uint32_t mat_types, unsigned long long* counters) {
     WfDev W = W0;
     const unsigned pblocks = PersistBlocks(c);
     for (int depth = 0; depth < depth_max; ++depth) {
@@ -1054,24 +1127,21 @@ static int WfBounceLoop(Ctx* c, const R& Rd, const WfDev& W0, int depth_max, int
         if (env) hipLaunchKernelGGL((k_wf_env<0, R>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
         TimerEnd(c);
         TimerBegin(c, kKernShade);
-        if (env) {
-            hipLaunchKernelGGL((k_wf_shade<0, R, true>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
-            hipLaunchKernelGGL((k_wf_shade<1, R, true>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
-            hipLaunchKernelGGL((k_wf_shade<2, R, true>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
-            hipLaunchKernelGGL((k_wf_shade<3, R, true>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
-        } else {
-            hipLaunchKernelGGL((k_wf_shade<0, R, false>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
-            hipLaunchKernelGGL((k_wf_shade<1, R, false>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
-            hipLaunchKernelGGL((k_wf_shade<2, R, false>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
-            hipLaunchKernelGGL((k_wf_shade<3, R, false>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
-        }
+        // a bin that no scene of the launch has a material for stays empty
+        const auto shade = [&](int m, void (*with_env)(R, WfDev), void (*without)(R, WfDev)) {
+            if (mat_types & (1u << m)) hipLaunchKernelGGL(env ? with_env : without, dim3(blocks), dim3(256), 0, c->stream, Rd, W);
+        };
+        shade(0, k_wf_shade<0, R, true>, k_wf_shade<0, R, false>);
+        shade(1, k_wf_shade<1, R, true>, k_wf_shade<1, R, false>);
+        shade(2, k_wf_shade<2, R, true>, k_wf_shade<2, R, false>);
+        shade(3, k_wf_shade<3, R, true>, k_wf_shade<3, R, false>);
         TimerEnd(c);
         TimerBegin(c, kKernTraceShadow);  // shadow and MIS rays
         hipLaunchKernelGGL((k_wf_trace_shadow_mis<STACK, R>), dim3(pblocks), dim3(256), 0, c->stream, Rd, W,
                            refill > 0 ? refill : kAutoRefill, kTraceChunks[1], kTraceChunks[2]);
         TimerEnd(c);
         TimerBegin(c, kKernOther);
-        if (env) hipLaunchKernelGGL((k_wf_env<1, R>), dim3(blocks), dim3(256), 0, c->stream, Rd, W);
+        if (env) hipLaunchKernelGGL((k_wf_env<1, R>), dim3((unsigned)(((uint64_t)W.part * kParts + 255) / 256)), dim3(256), 0, c->stream, Rd, W);
         hipLaunchKernelGGL((k_wf_resolve<R>), dim3(ResolveBlocks(n_slots)), dim3(256), 0, c->stream, Rd, W, n_slots);
         hipLaunchKernelGGL(k_wf_advance, dim3(1), dim3(64), 0, c->stream, W, counters);
         TimerEnd(c);
@@ -1118,8 +1188,7 @@ int WavefrontPass(Ctx* c, Scene* sc, const PathParams& P, const gy_render_params
     }
     if (sc->stats.max_depth + 1 > 64) return Fail(GY_ERR_UNSUPPORTED, "BVH deeper than the traversal stack");
     return WfBounceLoop<kStackLds>(c, Rd, W, p.max_depth, RefillOf(p.refill_threshold), p.ray_sort, blocks, (uint32_t)cap,
-                                   sc->dev.env.w > 0,
-                                   sc->film.counters);
+                                   sc->dev.env.w > 0, sc->mat_types, sc->film.counters);
 }
 
 // ---------------------------------------------------------------- light tracing
@@ -1209,10 +1278,9 @@ __global__ void __launch_bounds__(256) k_lt_start(SceneDev S, PathParams P, WfDe
         W.T[slot] = make_float4(T.x, T.y, T.z, __uint_as_float(st_pack(q.cursor, 1u, false, 0u)));
         W.idx[slot] = make_uint2((uint32_t)q.index, (uint32_t)(q.index >> 32));
     }
-    uint32_t* const qs[2] = {W.q[Q_SHADOW], W.q[Q_NEXT]};
-    uint32_t* const cs[2] = {&W.counts[Q_SHADOW * kCtrStride], &W.counts[Q_NEXT * kCtrStride]};
-    const bool ps[2] = {conn, valid};
-    block_push<2>(qs, cs, slot, ps);
+    if (valid) W.q[Q_NEXT][t] = slot;  // every path goes on
+    if (t == 0) W.counts[Q_NEXT * kCtrStride] = (uint32_t)n;
+    part_push(W, slot, conn, false);
 }
 
 // Trace's loop body after an intersection (integrator/LT.h:62-83) with the
@@ -1258,10 +1326,11 @@ __global__ void __launch_bounds__(256) k_lt_shade(SceneDev S, PathParams P, WfDe
             next = true;
         }
     }
-    uint32_t* const qs[2] = {W.q[Q_SHADOW], W.q[Q_NEXT]};
-    uint32_t* const cs[2] = {&W.counts[Q_SHADOW * kCtrStride], &W.counts[Q_NEXT * kCtrStride]};
-    const bool ps[2] = {conn, next};
-    block_push<2>(qs, cs, slot, ps);
+    part_push(W, slot, conn, false);
+    uint32_t* const qs[1] = {W.q[Q_NEXT]};
+    uint32_t* const cs[1] = {&W.counts[Q_NEXT * kCtrStride]};
+    const bool ps[1] = {next};
+    block_push<1>(qs, cs, slot, ps);
 }
 
 int LightTracingWavefront(Ctx* c, Scene* sc, const PathParams& P, const LightCamDev& C, int64_t n, float total, float* splat) {
@@ -1325,6 +1394,17 @@ int LightTracingWavefront(Ctx* c, Scene* sc, const PathParams& P, const LightCam
 // The whole batch: clear every entry's film, run the lane space in passes of
 // `lanes` paths (raygen + bounce loop to the largest depth), resolve every
 // entry's film.  No host round trip, so it is recorded into a graph once.
+// Paths with a pixel before global path index g (tile-padded entries hold lanes without one).
+static int64_t BatchValid(const Batch* b, int64_t g) {
+    for (const BatchEntry& en : b->entries) {
+        const int W = en.cam.width, H = en.cam.height;
+        if (g >= en.first + en.paths) continue;
+        const int64_t per_s = (int64_t)((W + 7) >> 3) * ((H + 7) >> 3) * 64, r = g - en.first, s = r / per_s;
+        return en.first_valid + s * W * H + tile_rank(W, H, r - s * per_s);
+    }
+    const BatchEntry& last = b->entries.back();
+    return last.first_valid + (int64_t)last.cam.width * last.cam.height * last.params.spp;
+}
 static int BatchSequence(Ctx* c, Batch* b) {
     const int64_t lanes = b->lanes;
     size_t used = 0;
@@ -1343,15 +1423,20 @@ static int BatchSequence(Ctx* c, Batch* b) {
     if (rc != GY_OK) return rc;
     const unsigned blocks = (unsigned)((lanes + 255) / 256);
     bool env = false;
-    for (auto& en : b->entries) env = env || en.scene->dev.env.w > 0;
+    uint32_t mat_types = 0;
+    for (auto& en : b->entries) {
+        env = env || en.scene->dev.env.w > 0;
+        mat_types |= en.scene->mat_types;
+    }
     for (int64_t base = 0; base < b->total_paths && rc == GY_OK; base += lanes) {
         const int64_t count = std::min(lanes, b->total_paths - base);
         hipLaunchKernelGGL(k_wf_reset, dim3(1), dim3(64), 0, c->stream, W);
         TimerBegin(c, kKernRaygen);
-        hipLaunchKernelGGL(k_wf_raygen_batch, dim3(blocks), dim3(256), 0, c->stream, W, Rd, base, count, lanes);
+        hipLaunchKernelGGL(k_wf_raygen_batch, dim3(blocks), dim3(256), 0, c->stream, W, Rd, base, count, lanes, BatchValid(b, base),
+                           (uint32_t)(BatchValid(b, base + count) - BatchValid(b, base)));
         TimerEnd(c);
         rc = CheckLaunch(c, "k_wf_raygen_batch");
-        if (rc == GY_OK) rc = WfBounceLoop<kStackLds>(c, Rd, W, b->depth_max, b->refill, b->ray_sort, blocks, (uint32_t)lanes, env, b->counters);
+        if (rc == GY_OK) rc = WfBounceLoop<kStackLds>(c, Rd, W, b->depth_max, b->refill, b->ray_sort, blocks, (uint32_t)lanes, env, mat_types, b->counters);
     }
     for (auto& en : b->entries)
         if (rc == GY_OK) rc = FilmResolveState(c, en.film, en.params.spp);
