@@ -198,11 +198,12 @@ __global__ void __launch_bounds__(256) k_count_visits(SceneDev S, const gy_ray* 
     wave_add_u64(&counters[1], nt);
 }
 
-// Five waves per SIMD, the most its LDS stack allows at 128 lanes (166 VGPRs
-// and three waves without the hint): 96 VGPRs with some spilled, 1.27x faster
-// on the 1.31M-triangle icosphere (108.6 -> 138.3 Mpaths/s).
-template <int STACK, int BLOCK, bool ENV, bool SPH>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
+// WAVES per SIMD: five (96 VGPRs, some spilled) for launches that fill the card,
+// 16.1 ms for 3.3M paths of depth 10 over 82k triangles against 16.6 at four,
+// 18.0 at three and 24.0 without the hint; three (no spills in the loop, which
+// wait on scratch memory) for launches that do not (kMegaSmallWaves).
+template <int STACK, int BLOCK, bool ENV, bool SPH, int WAVES = 5>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES)))
 k_pt_megakernel(SceneDev S, PathParams P, FilmDev F, int s0, int n_s,
                                                          unsigned long long* counters) {
     __shared__ uint32_t stack[kPathLds * BLOCK];
@@ -766,7 +767,7 @@ int ValidateRender(const gy_camera_desc* cam, const gy_render_params* p) {
     return GY_OK;
 }
 
-template <int STACK, int BLOCK, bool SPH>
+template <int STACK, int BLOCK, bool SPH, int WAVES = 5>
 int LaunchMegaT(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, int s0, int n_s, bool count, bool timed) {
     FilmDev F = FilmViewState(film);
     const int tilesX = (F.width + 7) >> 3, tilesY = (F.height + 7) >> 3;
@@ -782,21 +783,31 @@ int LaunchMegaT(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, i
     }
     if (timed) TimerBegin(c, kKernMega);
     if (sc->dev.env.w > 0)
-        hipLaunchKernelGGL((k_pt_megakernel<STACK, BLOCK, true, SPH>), dim3(blocks), dim3(BLOCK), 0, c->stream, sc->dev, P, F, s0, n_s, ctr);
+        hipLaunchKernelGGL((k_pt_megakernel<STACK, BLOCK, true, SPH, WAVES>), dim3(blocks), dim3(BLOCK), 0, c->stream, sc->dev, P, F, s0, n_s, ctr);
     else
-        hipLaunchKernelGGL((k_pt_megakernel<STACK, BLOCK, false, SPH>), dim3(blocks), dim3(BLOCK), 0, c->stream, sc->dev, P, F, s0, n_s, ctr);
+        hipLaunchKernelGGL((k_pt_megakernel<STACK, BLOCK, false, SPH, WAVES>), dim3(blocks), dim3(BLOCK), 0, c->stream, sc->dev, P, F, s0, n_s, ctr);
     if (timed) TimerEnd(c);
     return CheckLaunch(c, "k_pt_megakernel");
 }
 
 // The megakernel over one pass into `film` (the scene's own film, or the
 // no-alloc entry point's).  Scenes with spheres run the sphere instantiation
-// at 128 threads a block.
+// at 128 threads a block.  block 0 is automatic: 128 threads, or one wave a
+// block of the three-wave instantiation when the pass has no more waves than
+// that keeps resident; such a launch is a chain of latencies, and its waves
+// spread over twice the CUs (16,384 paths of depth 5: 197 -> 160 us).
+constexpr int kMegaSmallWaves = 3;
 int LaunchMegaFilm(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, int s0, int n_s, int block, bool count,
                    bool timed) {
     if (sc->dev.n_sph > 0)
         return sc->stack <= 64 ? LaunchMegaT<64, 128, true>(c, sc, film, P, s0, n_s, count, timed)
                                : LaunchMegaT<192, 128, true>(c, sc, film, P, s0, n_s, count, timed);
+    if (block == 0) {
+        const int64_t waves = (int64_t)((film.width + 7) >> 3) * ((film.height + 7) >> 3) * n_s;
+        if (!count && waves <= (int64_t)c->num_cu * 4 * kMegaSmallWaves)
+            return sc->stack <= 64 ? LaunchMegaT<64, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed)
+                                   : LaunchMegaT<192, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed);
+    }
     if (sc->stack <= 64) {
         if (block == 64) return LaunchMegaT<64, 64, false>(c, sc, film, P, s0, n_s, count, timed);
         if (block == 256) return LaunchMegaT<64, 256, false>(c, sc, film, P, s0, n_s, count, timed);
@@ -1353,7 +1364,7 @@ extern "C" int gy_render(gy_scene* s, const gy_camera_desc* cam, const gy_render
     (void)hipEventCreate(&t0);
     (void)hipEventCreate(&t1);
     (void)hipEventRecord(t0, c->stream);
-    int block = p->block_size > 0 ? p->block_size : 128;
+    const int block = p->block_size > 0 ? p->block_size : 0;
     // scenes with spheres render with the per-path kernels (same film)
     const bool wavefront = p->mode == GY_RENDER_WAVEFRONT && sc->dev.n_sph == 0;
     for (int s0 = 0; s0 < p->spp && rc == GY_OK; s0 += n_pass) {
@@ -1448,7 +1459,7 @@ extern "C" int gy_render_noalloc(gy_scene* s, const gy_camera_desc* cam, const g
     f.width = cam->width;
     f.height = cam->height;
     rc = FilmClear(c, f);
-    const int block = p->block_size > 0 ? p->block_size : 128;
+    const int block = p->block_size > 0 ? p->block_size : 0;
     for (int s0 = 0; s0 < p->spp && rc == GY_OK; s0 += n_pass) {
         const int n_s = std::min(n_pass, p->spp - s0);
         rc = LaunchMegaFilm(c, sc, f, P, s0, n_s, block, false, false);
