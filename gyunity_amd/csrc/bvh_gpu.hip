@@ -545,7 +545,8 @@ struct WideKids {
     uint32_t inner;  // interior children
 };
 __host__ __device__ inline float bits_float(uint32_t v) { return __builtin_bit_cast(float, v); }
-__host__ __device__ inline WideKids wide_open(const uint4* binary, uint32_t open) {
+// pad: added to every side of the boxes.
+__host__ __device__ inline WideKids wide_open(const uint4* binary, uint32_t open, float pad) {
     WideKids w;
     int n = 0, at = 0;
     while (true) {
@@ -558,7 +559,10 @@ __host__ __device__ inline WideKids wide_open(const uint4* binary, uint32_t open
             const int s = first ? at : n;
             if (s == n) ++n;
             first = false;
-            for (int k = 0; k < 6; ++k) w.box[s][k] = bits_float(q[6 * c + k]);
+            for (int k = 0; k < 3; ++k) {
+                w.box[s][k] = bits_float(q[6 * c + k]) - pad;
+                w.box[s][3 + k] = bits_float(q[6 * c + 3 + k]) + pad;
+            }
             w.ref[s] = q[12 + c];
             w.cnt[s] = q[14 + c];
         }
@@ -622,10 +626,10 @@ __host__ __device__ inline gyd::WideNode wide_make(const WideKids& w, uint32_t n
 // nodes of a level is not fixed; no result depends on it.  1.31M triangles:
 // 0.44M nodes from 1.31M.
 __global__ void __launch_bounds__(64) k_wide_level(const uint4* __restrict__ binary, gyd::WideNode* __restrict__ wide,
-                                                   uint32_t* __restrict__ src, uint32_t* __restrict__ ctr) {
+                                                   uint32_t* __restrict__ src, uint32_t* __restrict__ ctr, float pad) {
     const uint32_t end = ctr[2];
     for (uint32_t w = ctr[1] + blockIdx.x * 64 + threadIdx.x; w < end; w += gridDim.x * 64) {
-        const WideKids kids = wide_open(binary, src[w]);
+        const WideKids kids = wide_open(binary, src[w], pad);
         const uint32_t next = kids.inner ? atomicAdd(&ctr[0], kids.inner) : 0u;
         wide[w] = wide_make(kids, next);
         uint32_t i = next;
@@ -648,78 +652,68 @@ __global__ void k_wide_root(uint32_t* src, uint32_t* ctr) {
     ctr[3] = 0u;
 }
 
+constexpr uint32_t kWideHost = 1024;
+
+// The wide tree of the n binary nodes at `binary`, while they are still on the
+// device: built in `tmp` (room for n nodes) and `src` (n words), kept in an
+// allocation of its own size.  From the host's copy of the nodes it took their
+// upload (84 MB at 1.31M triangles) and four allocations more: 34 ms of a scene
+// creation that takes 120.
+int WideDevice(Ctx* c, const uint32_t* binary, int64_t n, int max_depth, float pad, void* tmp, uint32_t* src, uint32_t* ctr,
+               BVHBuild* out) {
+    const unsigned blocks = (unsigned)std::min<int64_t>((n + 63) / 64, 4096);
+    hipLaunchKernelGGL(k_wide_root, dim3(1), dim3(64), 0, c->stream, src, ctr);
+    for (int l = 0; l <= max_depth; ++l) {
+        hipLaunchKernelGGL(k_wide_level, dim3(blocks), dim3(64), 0, c->stream, (const uint4*)binary, (gyd::WideNode*)tmp, src, ctr, pad);
+        hipLaunchKernelGGL(k_wide_advance, dim3(1), dim3(64), 0, c->stream, ctr);
+    }
+    int rc = CheckLaunch(c, "wide bvh");
+    if (rc != GY_OK) return rc;
+    uint32_t h[4] = {0, 0, 0, 0};
+    hipError_t e = hipMemcpyAsync(h, ctr, 16, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return HipFail(e, "wide bvh");
+    if (h[1] != h[2]) return Fail(GY_ERR_DEVICE, "wide bvh: levels left over");
+    rc = DevAlloc(c, &out->wide, (size_t)h[0] * sizeof(gyd::WideNode));
+    if (rc != GY_OK) return rc;
+    e = hipMemcpyAsync(out->wide, tmp, (size_t)h[0] * sizeof(gyd::WideNode), hipMemcpyDeviceToDevice, c->stream);
+    if (e != hipSuccess) {
+        DevFree(out->wide);
+        out->wide = nullptr;
+        return HipFail(e, "wide bvh copy");
+    }
+    out->n_wide = h[0];
+    out->wide_depth = (int32_t)h[3];
+    return GY_OK;
+}
+
 }  // namespace
 
-// Small trees are collapsed on the host: up to kWideHost nodes (a few tens of
-// microseconds) the device's launches, allocations and read-back (0.2 ms) would
-// cost more.
-constexpr int64_t kWideHost = 1024;
-static int BuildWideHost(Ctx* c, const std::vector<uint32_t>& nodes, void** wide, int64_t* n_wide, int* depth) {
+// The wide tree of a binary tree on the host (padded boxes): the host's builds,
+// and the device's up to kWideHost nodes (a few tens of microseconds; the
+// device's launches and read-back take 0.2 ms).
+int BuildWideHost(Ctx* c, BVHBuild* b) {
     std::vector<gyd::WideNode> out;
     std::vector<uint32_t> src(1, 0u);
-    const uint4* binary = reinterpret_cast<const uint4*>(nodes.data());
+    const uint4* binary = reinterpret_cast<const uint4*>(b->nodes.data());
     size_t begin = 0;
-    *depth = 0;
+    b->wide_depth = 0;
     while (begin < src.size()) {  // a level
         const size_t end = src.size();
         for (; begin < end; ++begin) {
-            const WideKids kids = wide_open(binary, src[begin]);
+            const WideKids kids = wide_open(binary, src[begin], 0.f);
             out.push_back(wide_make(kids, (uint32_t)src.size()));
             for (int s = 0; s < kids.n; ++s)
                 if (kids.cnt[s] == 0) src.push_back(kids.ref[s]);
         }
-        ++*depth;
+        ++b->wide_depth;
     }
-    *n_wide = (int64_t)out.size();
-    return Upload(c, wide, out.data(), out.size() * sizeof(gyd::WideNode));
-}
-
-int BuildWideBVH(Ctx* c, const std::vector<uint32_t>& nodes, int max_depth, void** wide, int64_t* n_wide, int* depth) {
-    const int64_t n_binary = (int64_t)(nodes.size() / 16);
-    if (n_binary <= kWideHost) return BuildWideHost(c, nodes, wide, n_wide, depth);
-    *wide = nullptr;
-    void *binary = nullptr, *tmp = nullptr, *src = nullptr, *ctr = nullptr;
-    int rc = Upload(c, &binary, nodes.data(), nodes.size() * 4);
-    // each wide node stands for a binary node of its own
-    if (rc == GY_OK) rc = DevAlloc(c, &tmp, (size_t)n_binary * sizeof(gyd::WideNode));
-    if (rc == GY_OK) rc = DevAlloc(c, &src, (size_t)n_binary * 4);
-    if (rc == GY_OK) rc = DevAlloc(c, &ctr, 16);
-    uint32_t h[4] = {0, 0, 0, 0};
-    if (rc == GY_OK) {
-        const unsigned blocks = (unsigned)std::min<int64_t>((n_binary + 63) / 64, 4096);
-        hipLaunchKernelGGL(k_wide_root, dim3(1), dim3(64), 0, c->stream, (uint32_t*)src, (uint32_t*)ctr);
-        for (int l = 0; l <= max_depth; ++l) {
-            hipLaunchKernelGGL(k_wide_level, dim3(blocks), dim3(64), 0, c->stream, (const uint4*)binary, (gyd::WideNode*)tmp, (uint32_t*)src, (uint32_t*)ctr);
-            hipLaunchKernelGGL(k_wide_advance, dim3(1), dim3(64), 0, c->stream, (uint32_t*)ctr);
-        }
-        rc = CheckLaunch(c, "wide bvh");
-        hipError_t e = hipMemcpyAsync(h, ctr, 16, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (rc == GY_OK && e != hipSuccess) rc = HipFail(e, "wide bvh");
-        if (rc == GY_OK && h[1] != h[2]) rc = Fail(GY_ERR_DEVICE, "wide bvh: levels left over");
-    }
-    if (rc == GY_OK) rc = DevAlloc(c, wide, (size_t)h[0] * sizeof(gyd::WideNode));
-    if (rc == GY_OK) {
-        hipError_t e = hipMemcpyAsync(*wide, tmp, (size_t)h[0] * sizeof(gyd::WideNode), hipMemcpyDeviceToDevice, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (e != hipSuccess) rc = HipFail(e, "wide bvh copy");
-    }
-    DevFree(binary);
-    DevFree(tmp);
-    DevFree(src);
-    DevFree(ctr);
-    if (rc != GY_OK) {
-        DevFree(*wide);
-        *wide = nullptr;
-        return rc;
-    }
-    *n_wide = h[0];
-    *depth = (int)h[3];
-    return GY_OK;
+    b->n_wide = (int64_t)out.size();
+    return Upload(c, &b->wide, out.data(), out.size() * sizeof(gyd::WideNode));
 }
 
 // Build on the device, then copy nodes and leaf order back for the scene upload.
-int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, BVHBuild* out) {
+int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, float pad, BVHBuild* out) {
     if (max_leaf < 1) max_leaf = 1;
     if (max_leaf > 15) max_leaf = 15;
     if (n_tri <= 2 * kSmall) {
@@ -846,8 +840,16 @@ int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, BVHBui
     if (e == hipSuccess) e = hipMemcpyAsync(out->tri_order.data(), B.idx[cur], n * 4, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return fail(e, "bvh download");
-    DevFree(base);
     out->max_depth = (int32_t)h[3];
+    if (nn > kWideHost) {
+        // the triangles and their bounds (68 bytes each) are done with: a node
+        // takes 64, and there are fewer nodes than triangles
+        if ((size_t)nn * sizeof(gyd::WideNode) > o_idx0 - o_pos || (size_t)nn > (size_t)n) rc = Fail(GY_ERR_DEVICE, "wide bvh: more nodes than triangles");
+        else rc = WideDevice(c, B.nodes, nn, out->max_depth, pad, base + o_pos, (uint32_t*)B.tid[0], acc, out);
+        (void)hipStreamSynchronize(c->stream);
+    }
+    DevFree(base);
+    if (rc != GY_OK) return rc;
     out->n_leaves = h[4];
     out->max_leaf = max_leaf;
     out->sah_cost = BVHSahCost(*out);

@@ -87,6 +87,10 @@ struct BVHBuild {
     int64_t n_leaves = 0;
     int32_t max_leaf = 0;
     double sah_cost = 0;
+    // the traversal tree (gyd::WideNode records on the device), and its levels
+    void* wide = nullptr;
+    int64_t n_wide = 0;
+    int32_t wide_depth = 0;
 };
 constexpr uint32_t kEmptyRef = 0xffffffffu;
 // Host binned-SAH build over triangle bounds.

@@ -510,9 +510,15 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     const int leaf = bvh.max_leaf_size > 0 ? bvh.max_leaf_size : 4;
     int rc = GY_OK;
     BVHBuild b;
+    // Pad every child box outward so that the traversal never rejects a box
+    // containing a triangle the triangle test accepts (rounding in that test
+    // can place an accepted hit slightly outside the triangle).
+    float ext = 0.f;
+    for (size_t i = 0; i < (size_t)d.n_tri * 9; ++i) ext = std::max(ext, std::fabs(d.pos[i]));
+    const float pad = 4e-6f * (1.f + ext);
     auto tb0 = std::chrono::steady_clock::now();
     if (bvh.builder == 0) {
-        rc = BuildBVHDevice(c, d.pos, d.n_tri, leaf, &b);
+        rc = BuildBVHDevice(c, d.pos, d.n_tri, leaf, pad, &b);
         if (rc != GY_OK) {
             delete sc;
             return rc;
@@ -527,16 +533,11 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     sc->stats.max_depth = b.max_depth;
     sc->stats.max_leaf_size = b.max_leaf;
     sc->stats.sah_cost = b.sah_cost;
+    sc->d_nodes = b.wide;
     if (b.max_depth + 1 > 64) {
-        delete sc;
+        SceneFree(sc);
         return Fail(GY_ERR_UNSUPPORTED, "BVH deeper than the 64-entry traversal stack");
     }
-    // Pad every child box outward so that the traversal never rejects a box
-    // containing a triangle the triangle test accepts (rounding in that test
-    // can place an accepted hit slightly outside the triangle).
-    float ext = 0.f;
-    for (size_t i = 0; i < (size_t)d.n_tri * 9; ++i) ext = std::max(ext, std::fabs(d.pos[i]));
-    const float pad = 4e-6f * (1.f + ext);
     for (size_t nidx = 0; nidx < b.nodes.size() / 16; ++nidx) {
         uint32_t* nd = &b.nodes[nidx * 16];
         for (int s = 0; s < 2; ++s) {
@@ -577,16 +578,12 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     if ((rc = Upload(c, &p, shade.data(), shade.size() * sizeof(float4))) != GY_OK) goto fail;
     sc->d_shade = p;
     sc->dev.shade = (const float4*)p;
-    {
-        int64_t n_wide = 0;
-        int depth = 0;
-        if ((rc = BuildWideBVH(c, b.nodes, b.max_depth, &p, &n_wide, &depth)) != GY_OK) goto fail;
-        sc->d_nodes = p;
-        sc->dev.nodes = (const WideNode*)p;
-        sc->dev.n_nodes = (int32_t)n_wide;
-        // the end mark, and at most three children of each node on a path
-        sc->stack = 1 + 3 * depth <= kStackSmall ? kStackSmall : kStackLarge;
-    }
+    if (!b.wide && (rc = BuildWideHost(c, &b)) != GY_OK) goto fail;
+    sc->d_nodes = b.wide;
+    sc->dev.nodes = (const WideNode*)b.wide;
+    sc->dev.n_nodes = (int32_t)b.n_wide;
+    // the end mark, and at most three children of each node on a path
+    sc->stack = 1 + 3 * b.wide_depth <= kStackSmall ? kStackSmall : kStackLarge;
     if ((rc = Upload(c, &p, d.mats, (size_t)d.n_mat * GY_MAT_WORDS * 4)) != GY_OK) goto fail;
     sc->d_mats = p;
     sc->dev.mats = (const uint32_t*)p;

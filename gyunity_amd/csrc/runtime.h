@@ -189,9 +189,8 @@ int BatchRender(Ctx* c, Batch* b);
 int BatchAdjoint(Ctx* c, Batch* b, const float* dimages, float* grad_tex, float* grad_le);
 int BatchImages(Ctx* c, Batch* b, float* images);
 // GPU binned-SAH BVH build (bvh_gpu.hip).
-int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, BVHBuild* out);
-// The traversal tree of a binary tree (bvh_gpu.hip): n_wide WideNode records on
-// the device in *wide, `depth` levels.
-int BuildWideBVH(Ctx* c, const std::vector<uint32_t>& nodes, int max_depth, void** wide, int64_t* n_wide, int* depth);
+int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, float pad, BVHBuild* out);
+// The wide tree of a binary tree on the host (padded boxes) into b->wide.
+int BuildWideHost(Ctx* c, BVHBuild* b);
 
 }  // namespace gy

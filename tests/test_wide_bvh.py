@@ -113,7 +113,7 @@ def brute_force(tri, rays):
             np.where(hit, b2[at], f(0)), hit.astype(np.int32))
 
 
-CASES = [("random", n) for n in (1, 2, 3, 4, 5, 16, 17, 129, 900)] + [("chain", 60), ("chain", 150), ("flat", 300), ("far", 300),
+CASES = [("random", n) for n in (1, 2, 3, 4, 5, 16, 17, 129, 900)] + [("chain", 60), ("chain", 150), ("flat", 300), ("far", 300), 
                                                                          ("overlap", 20000)]
 
 
@@ -152,3 +152,19 @@ def test_deep_stacks_render_alike_in_both_forms(gpu_ctx, kind, n):
             films.append(sc.render(cam, g.render_params(4, 4, mode=mode)))
     assert np.array_equal(films[0][0], films[1][0], equal_nan=True) and films[0][0].sum() > 0
     assert np.array_equal(films[0][1], films[1][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,n", [("random", 64), ("random", 3000), ("chain", 150)])
+def test_both_builders_trees_give_the_same_hits(gpu_ctx, kind, n):
+    # the device collapses its own binary trees of more than 1024 nodes, the
+    # host the smaller ones and those it built
+    rng = np.random.default_rng(n)
+    tri = soup(kind, n, rng)
+    rays = rays_for(tri, 4000, rng, 4.0)
+    found = []
+    for builder in (0, 1):
+        with g.Scene(gpu_ctx, scene(tri), builder=builder) as sc:
+            found.append((sc.trace_closest(rays), sc.trace_any(rays)))
+    assert found[0][0].tobytes() == found[1][0].tobytes()
+    assert np.array_equal(found[0][1], found[1][1])
