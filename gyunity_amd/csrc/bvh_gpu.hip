@@ -598,12 +598,19 @@ __host__ __device__ inline gyd::WideNode wide_make(const WideKids& w, uint32_t n
             lo = fminf(lo, w.box[s][k]);
             hi = fmaxf(hi, w.box[s][3 + k]);
         }
-        const float step = fmaxf((hi - lo) * (1.f / 250.f), 1e-30f);
-        o.org[k] = lo - 2.f * step;
+        // beyond 1e11 (or infinite, or NaN) a step times a ray's 1 / direction
+        // can leave FP32's range; the axis then takes part in no decision: the
+        // children's planes lie further out than any that FP32 can test
+        const bool open = !(hi - lo <= 1e11f);
+        const float step = open ? 1e30f : fmaxf((hi - lo) * (1.f / 250.f), 1e-30f);
+        o.org[k] = open ? -1.25e32f : lo - 2.f * step;
         o.scale[k] = step * 16777216.f;
         for (int s = 0; s < 4; ++s) {
             int mn = 255, mx = 0;  // absent: inverted
-            if (s < w.n) {
+            if (s < w.n && open) {
+                mn = 0;
+                mx = 255;
+            } else if (s < w.n) {
                 mn = (int)floor(((double)w.box[s][k] - (double)o.org[k]) / (double)step - 0.0078125);
                 mx = (int)ceil(((double)w.box[s][3 + k] - (double)o.org[k]) / (double)step + 0.0078125);
                 mn = mn < 0 ? 0 : (mn > 255 ? 255 : mn);

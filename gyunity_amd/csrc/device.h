@@ -480,7 +480,7 @@ GY_D void trav_init(Trav& t, V3 o, V3 d, float tmin, float tmax) {
     t.ti = v3(trav_inv(d.x, lim), trav_inv(d.y, lim), trav_inv(d.z, lim));
     // directions so short or long that the distances leave FP32's range: every
     // box is entered (0 * plane + 0), which is slow and loses nothing
-    if (m != 0.f && !(m > 1e-18f && m < 1e18f)) t.ti = v3(0.f, 0.f, 0.f);
+    if (m != 0.f && !(m > 1e-10f && m < 1e18f)) t.ti = v3(0.f, 0.f, 0.f);
     t.to = v3(-(o.x * t.ti.x), -(o.y * t.ti.y), -(o.z * t.ti.z));
     t.sx = t.ti.x < 0.f ? kNearMax : kNearMin;
     t.sy = t.ti.y < 0.f ? kNearMax : kNearMin;

@@ -25,6 +25,10 @@ def soup(kind, n, rng):
         d = rng.uniform(-0.05, 0.05, (n, 3, 3))
         d[..., 2] = 0
         return (c + d).astype(np.float32)
+    if kind == "wall":  # one triangle so large that the axes of the nodes above it take no part
+        tri = soup("random", n, rng)
+        tri[n // 2] = 1e12 * np.array([[-1, -1, -0.5], [3, -1, -0.5], [-1, 3, -0.5]])
+        return tri
     assert kind == "far"  # 300 away from the origin
     return (soup("random", n, rng).astype(np.float64) + 300.0).astype(np.float32)
 
@@ -42,6 +46,7 @@ def scene(tri, lights=1):
 
 
 def rays_for(tri, n, rng, far=40.0):
+    tri = tri[np.abs(tri).max((1, 2)) < 1e9]  # rays around and to the triangles of ordinary size
     lo, hi = tri.reshape(-1, 3).min(0).astype(np.float64), tri.reshape(-1, 3).max(0).astype(np.float64)
     ext = np.maximum(hi - lo, 0.1)
     target = tri[rng.integers(0, tri.shape[0], n)].astype(np.float64)
@@ -113,7 +118,7 @@ def brute_force(tri, rays):
             np.where(hit, b2[at], f(0)), hit.astype(np.int32))
 
 
-CASES = [("random", n) for n in (1, 2, 3, 4, 5, 16, 17, 129, 900)] + [("chain", 60), ("chain", 150), ("flat", 300), ("far", 300), 
+CASES = [("random", n) for n in (1, 2, 3, 4, 5, 16, 17, 129, 900)] + [("chain", 60), ("chain", 150), ("flat", 300), ("far", 300), ("wall", 300),
                                                                          ("overlap", 20000)]
 
 
@@ -155,7 +160,7 @@ def test_deep_stacks_render_alike_in_both_forms(gpu_ctx, kind, n):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind,n", [("random", 64), ("random", 3000), ("chain", 150)])
+@pytest.mark.parametrize("kind,n", [("random", 64), ("random", 3000), ("chain", 150), ("wall", 300)])
 def test_both_builders_trees_give_the_same_hits(gpu_ctx, kind, n):
     # the device collapses its own binary trees of more than 1024 nodes, the
     # host the smaller ones and those it built
