@@ -49,12 +49,6 @@ int Fill32(Ctx* c, void* p, uint32_t v, int64_t n) {
     return e == hipSuccess ? GY_OK : HipFail(e, "fill kernel");
 }
 
-int FillF4(Ctx* c, float4* p, int64_t n) {
-    if (n <= 0) return GY_OK;
-    hipLaunchKernelGGL(k_fill_f4, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, p, n);
-    return CheckLaunch(c, "fill");
-}
-
 int DevAlloc(Ctx* c, void** p, size_t bytes) {
     if (c->fault == GY_FAULT_ALLOC) {
         c->fault = GY_FAULT_NONE;
@@ -285,44 +279,8 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
 // scheduling.
 __global__ void k_film_accumulate(FilmDev F, int n_s) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int W = F.width, H = F.height;
-    const int64_t WH = (int64_t)W * H;
-    if (p >= WH) return;
-    const int x = (int)(p % W), y = (int)(p / W);
-    // bit b = (dy + 1) * 3 + dx + 1: the source pixel (x - dx, y - dy) has border samples
-    uint32_t nb = 0;
-    int64_t src[9];
-    for (int b = 0; b < 9; ++b) {
-        const int dx = b % 3 - 1, dy = b / 3 - 1;
-        int sx = x - dx, sy = y - dy;
-        sx = sx < 0 ? sx + W : (sx >= W ? sx - W : sx);
-        sy = sy < 0 ? sy + H : (sy >= H ? sy - H : sy);
-        src[b] = (int64_t)sy * W + sx;
-        if (b != 4 && F.border[src[b]]) nb |= 1u << b;
-    }
-    const bool own_border = F.border[p] != 0u;
-    float4 acc = F.film[p];
-    for (int s = 0; s < n_s; ++s) {
-        const int64_t base = (int64_t)s * WH;
-        const float4 e = F.pass[base + p];
-        if (own_border ? (((uint32_t)e.w & kFilmOwn) != 0u) : (e.w != 0.f)) {
-            acc.w += 1.0f;
-            acc.x = acc.x + e.x;
-            acc.y = acc.y + e.y;
-            acc.z = acc.z + e.z;
-        }
-        for (uint32_t m = nb; m != 0u; m &= m - 1u) {
-            const int b = __builtin_ctz(m);
-            const float4 q = F.pass[base + src[b]];
-            if (((uint32_t)q.w >> b) & 1u) {
-                acc.w += 1.0f;
-                acc.x = acc.x + q.x;
-                acc.y = acc.y + q.y;
-                acc.z = acc.z + q.z;
-            }
-        }
-    }
-    F.film[p] = acc;
+    if (p >= (int64_t)F.width * F.height) return;
+    F.film[p] = film_sum(F, p, n_s, F.film[p]);
 }
 
 // ------------------------------------------------------------------ launch helpers

@@ -383,6 +383,46 @@ __device__ inline void film_record(const FilmDev& F, int64_t slot, int px, int p
     F.pass[slot] = make_float4(L.x, L.y, L.z, (float)film_mark(F, px, py, fx, fy));
 }
 
+// Pixel p's sum: acc and the pass's samples (n_s a pixel) whose footprints hold it, sample by sample.
+__device__ inline float4 film_sum(const FilmDev& F, int64_t p, int n_s, float4 acc) {
+    const int W = F.width, H = F.height;
+    const int64_t WH = (int64_t)W * H;
+    const int x = (int)(p % W), y = (int)(p / W);
+    // bit b = (dy + 1) * 3 + dx + 1: the source pixel (x - dx, y - dy) has border samples
+    uint32_t nb = 0;
+    int64_t src[9];
+    for (int b = 0; b < 9; ++b) {
+        const int dx = b % 3 - 1, dy = b / 3 - 1;
+        int sx = x - dx, sy = y - dy;
+        sx = sx < 0 ? sx + W : (sx >= W ? sx - W : sx);
+        sy = sy < 0 ? sy + H : (sy >= H ? sy - H : sy);
+        src[b] = (int64_t)sy * W + sx;
+        if (b != 4 && F.border[src[b]]) nb |= 1u << b;
+    }
+    const bool own_border = F.border[p] != 0u;
+    for (int s = 0; s < n_s; ++s) {
+        const int64_t base = (int64_t)s * WH;
+        const float4 e = F.pass[base + p];
+        if (own_border ? (((uint32_t)e.w & kFilmOwn) != 0u) : (e.w != 0.f)) {
+            acc.w += 1.0f;
+            acc.x = acc.x + e.x;
+            acc.y = acc.y + e.y;
+            acc.z = acc.z + e.z;
+        }
+        for (uint32_t m = nb; m != 0u; m &= m - 1u) {
+            const int b = __builtin_ctz(m);
+            const float4 q = F.pass[base + src[b]];
+            if (((uint32_t)q.w >> b) & 1u) {
+                acc.w += 1.0f;
+                acc.x = acc.x + q.x;
+                acc.y = acc.y + q.y;
+                acc.z = acc.z + q.z;
+            }
+        }
+    }
+    return acc;
+}
+
 __device__ inline void record_sample(const FilmDev& F, int s_local, int px, int py, float fx, float fy, V3 L) {
     const int64_t WH = (int64_t)F.width * F.height;
     film_record(F, (int64_t)s_local * WH + (int64_t)py * F.width + px, px, py, fx, fy, L);

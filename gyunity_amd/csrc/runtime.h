@@ -116,7 +116,6 @@ int Upload(Ctx* c, void** p, const void* src, size_t bytes);
 void DevFree(void* p);
 int Grow(Ctx* c, DevBuf* b, size_t bytes);
 int Fill32(Ctx* c, void* p, uint32_t v, int64_t n);
-int FillF4(Ctx* c, float4* p, int64_t n);  // zero n float4
 int CheckLaunch(Ctx* c, const char* what);
 void TimerBegin(Ctx* c, int cat);
 void TimerEnd(Ctx* c);
