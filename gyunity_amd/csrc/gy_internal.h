@@ -74,7 +74,7 @@ struct LightCameraRT {
 };
 int BuildLightCamera(const gy_camera_desc& d, LightCameraRT* out);
 
-// BVH in the device layout: 16 words per node.
+// The binary BVH, from which the wide traversal tree is made: 16 words per node.
 //   words 0-5   child 0 AABB (min xyz, max xyz)
 //   words 6-11  child 1 AABB
 //   word 12/13  child 0/1 reference: node index (interior), first triangle (leaf),

@@ -11,7 +11,7 @@
 //
 // Every FP32 operation is the megakernel's, in the same order, so a render is
 // bit-identical to the megakernel's.  Queues are compacted with a wavefront
-// ballot and one atomic per wave; launch grids are fixed by the pass capacity
+// ballot and one atomic per workgroup; launch grids are fixed by the pass capacity
 // and kernels read their queue length from device memory, so a bounce needs no
 // host round trip.
 //
@@ -21,7 +21,7 @@
 //                sample budget, film) in a device table, so paths of many
 //                renders of uneven size share one lane space, one set of
 //                queues and the same persistent trace waves, which steal queue
-//                entries 64 at a time whatever render they belong to.
+//                entries whatever render they belong to.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -289,10 +289,9 @@ __global__ void __launch_bounds__(256) k_wf_raygen(WfDev W, PathParams P, FilmDe
 // The films of a batch: one thread a pixel of the entries' concatenated images
 // (image_off), so that the border flags of all entries are cleared in one
 // launch and their samples summed in one.  Launch-bound before: five launches
-// an entry, each too small to fill the card (16 entries of
-// 256 x 256, 16 samples: 12.1 -> 11.8 ms a render).  The films
-// need no clearing, since a batch sums all samples of a pixel at once, and the
-// flags only at the start.
+// an entry, each too small to fill the card (16 entries of 256 x 256, 16
+// samples: 12.1 -> 11.8 ms a render).  The films need no clearing, since a
+// batch sums all samples of a pixel at once, and the flags only at the start.
 __device__ inline const BatchEntryDev& batch_pixel(const ManyRenders& R, int64_t px, int64_t* p) {
     int lo = 0, hi = R.n - 1;  // last entry whose image begins at or before px
     while (lo < hi) {

@@ -239,7 +239,8 @@ int gy_vpt_li_samples(gy_scene* scene, const gy_camera_desc* cam, const gy_rende
 int gy_scene_stats_get(gy_scene* scene, gy_scene_stats* out);
 /* The context a scene was created on. */
 int gy_scene_context(gy_scene* scene, gy_context** ctx);
-/* Copy the device BVH back: nodes (n_nodes*16 words) and leaf triangle order. */
+/* Copy the binary BVH that the traversal tree is made from: nodes (n_nodes*16
+   words), padded boxes, and leaf triangle order. */
 int gy_scene_bvh_download(gy_scene* scene, uint32_t* nodes, int64_t max_nodes, int32_t* tri_order, int64_t max_tris);
 
 /* ---- ray queries (Scene::Intersect, visual/Scene.h:83-89 ->
