@@ -31,7 +31,7 @@ GY_SAMPLER_HALTON = 1
 GY_RAY_SORT_NONE = 0
 GY_RAY_SORT_OCTANT = 1
 GY_RAY_SORT_OCTANT_LOCAL = 2
-FAULT_NONE, FAULT_ALLOC, FAULT_LAUNCH, FAULT_SCENE = 0, 1, 2, 3
+FAULT_NONE, FAULT_ALLOC, FAULT_LAUNCH, FAULT_SCENE, FAULT_SYNC = 0, 1, 2, 3, 4
 
 
 class SceneDesc(C.Structure):

@@ -853,7 +853,14 @@ int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, float 
         // takes 64, and there are fewer nodes than triangles
         if ((size_t)nn * sizeof(gyd::WideNode) > o_idx0 - o_pos || (size_t)nn > (size_t)n) rc = Fail(GY_ERR_DEVICE, "wide bvh: more nodes than triangles");
         else rc = WideDevice(c, B.nodes, nn, out->max_depth, pad, base + o_pos, (uint32_t*)B.tid[0], acc, out);
-        (void)hipStreamSynchronize(c->stream);
+        // the copy out of `base` is part of the build: traversal follows the
+        // tree's indices without bounds checks
+        const int sync = StreamSync(c, "wide bvh copy");
+        if (rc == GY_OK) rc = sync;
+        if (rc != GY_OK) {
+            DevFree(out->wide);
+            out->wide = nullptr;
+        }
     }
     DevFree(base);
     if (rc != GY_OK) return rc;

@@ -98,6 +98,15 @@ int CheckLaunch(Ctx* c, const char* what) {
     return e == hipSuccess ? GY_OK : HipFail(e, what);
 }
 
+int StreamSync(Ctx* c, const char* what) {
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (c->fault == GY_FAULT_SYNC) {
+        c->fault = GY_FAULT_NONE;
+        return Fail(GY_ERR_INJECTED, std::string("injected failure of ") + what);
+    }
+    return e == hipSuccess ? GY_OK : HipFail(e, what);
+}
+
 // Timed region on the context stream: events recorded around each launch of a
 // kernel category and summed after the stream synchronises.
 void TimerBegin(Ctx* c, int cat) {
@@ -919,7 +928,7 @@ extern "C" int gy_device_name(gy_context* ctx, char* buf, int len) {
 
 extern "C" int gy_debug_inject_fault(gy_context* ctx, int kind) {
     if (!ctx) return Fail(GY_ERR_INVALID, "gy_debug_inject_fault: null context");
-    if (kind < GY_FAULT_NONE || kind > GY_FAULT_SCENE) return Fail(GY_ERR_INVALID, "gy_debug_inject_fault: unknown kind");
+    if (kind < GY_FAULT_NONE || kind > GY_FAULT_SYNC) return Fail(GY_ERR_INVALID, "gy_debug_inject_fault: unknown kind");
     reinterpret_cast<Ctx*>(ctx)->fault = kind;
     return GY_OK;
 }

@@ -117,6 +117,7 @@ void DevFree(void* p);
 int Grow(Ctx* c, DevBuf* b, size_t bytes);
 int Fill32(Ctx* c, void* p, uint32_t v, int64_t n);
 int CheckLaunch(Ctx* c, const char* what);
+int StreamSync(Ctx* c, const char* what);  // wait for the stream; its failure, or an injected one
 void TimerBegin(Ctx* c, int cat);
 void TimerEnd(Ctx* c);
 void TimersCollect(Ctx* c);

@@ -459,8 +459,10 @@ int gy_adjoint_emission_device(gy_scene* scene, const gy_camera_desc* cam, const
 float gy_ggx_dlogf_dalpha(float alpha, const float* wo, const float* wi);
 float gy_dalpha_droughness(float roughness);
 
-/* ---- failure injection (host-forced, for tests) --------------------------- */
-enum { GY_FAULT_NONE = 0, GY_FAULT_ALLOC = 1, GY_FAULT_LAUNCH = 2, GY_FAULT_SCENE = 3 };
+/* ---- failure injection (host-forced, for tests) ---------------------------
+   The next allocation, kernel launch, scene creation, or wait for a traversal
+   tree built on the device fails. */
+enum { GY_FAULT_NONE = 0, GY_FAULT_ALLOC = 1, GY_FAULT_LAUNCH = 2, GY_FAULT_SCENE = 3, GY_FAULT_SYNC = 4 };
 int gy_debug_inject_fault(gy_context* ctx, int kind);
 
 #ifdef __cplusplus

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import gyunity_amd as g
+from gyunity_amd._lib import FAULT_SYNC, GY_ERR_INJECTED
 
 def soup(kind, n, rng):
     """n triangles, (n, 3, 3) float32."""
@@ -173,3 +174,17 @@ def test_both_builders_trees_give_the_same_hits(gpu_ctx, kind, n):
             found.append((sc.trace_closest(rays), sc.trace_any(rays)))
     assert found[0][0].tobytes() == found[1][0].tobytes()
     assert np.array_equal(found[0][1], found[1][1])
+
+
+@pytest.mark.gpu
+def test_a_tree_whose_copy_failed_makes_no_scene(gpu_ctx):
+    # the device's tree is copied out of the build's workspace last; traversal
+    # follows its indices without bounds checks
+    sa, _, _ = g.generate_scene(g.GY_SCENE_ICOSPHERE_GGX, 1, 6)
+    gpu_ctx.inject_fault(FAULT_SYNC)
+    with pytest.raises(g.GyError) as e:
+        g.Scene(gpu_ctx, sa)
+    assert e.value.code == GY_ERR_INJECTED
+    rays = rays_for(sa.pos.reshape(-1, 3, 3), 1000, np.random.default_rng(0))
+    with g.Scene(gpu_ctx, sa) as sc:
+        assert (sc.trace_closest(rays)["prim"] >= 0).mean() > 0.2
