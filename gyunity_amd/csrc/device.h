@@ -472,6 +472,7 @@ GY_D float trav_inv(float d, float lim) {
     const float i = __builtin_amdgcn_rcpf(d);
     return fabsf(i) > lim ? copysignf(lim, i) : i;  // NaN stays NaN: that axis culls nothing
 }
+constexpr float kDirMin = 1e-10f, kDirMax = 1e18f;
 GY_D void trav_init(Trav& t, V3 o, V3 d, float tmin, float tmax) {
     t.o = o;
     t.d = d;
@@ -480,7 +481,7 @@ GY_D void trav_init(Trav& t, V3 o, V3 d, float tmin, float tmax) {
     t.ti = v3(trav_inv(d.x, lim), trav_inv(d.y, lim), trav_inv(d.z, lim));
     // directions so short or long that the distances leave FP32's range: every
     // box is entered (0 * plane + 0), which is slow and loses nothing
-    if (m != 0.f && !(m > 1e-10f && m < 1e18f)) t.ti = v3(0.f, 0.f, 0.f);
+    if (m != 0.f && !(m > kDirMin && m < kDirMax)) t.ti = v3(0.f, 0.f, 0.f);
     t.to = v3(-(o.x * t.ti.x), -(o.y * t.ti.y), -(o.z * t.ti.z));
     t.sx = t.ti.x < 0.f ? kNearMax : kNearMin;
     t.sy = t.ti.y < 0.f ? kNearMax : kNearMin;
@@ -668,17 +669,31 @@ struct SpillPrivate {
     GY_D void put(uint32_t i, uint32_t e) const { a[i] = e; }
     GY_D uint32_t get(uint32_t i) const { return a[i]; }
 };
-template <bool ANY, int STACK, bool COUNT = false, bool SPH = false>
+// The exponent k for which a ray with direction d * 2^k and distances * 2^-k has
+// a direction of length about 1, or 0 where the slab test takes the direction
+// as it is (trav_init enters every box for others: 65,536 rays through 5,132
+// triangles took 4.2 ms in place of 0.22).  Powers of two change no rounding of
+// the triangle test, whose products stay in FP32's range down to 1e-24 and up
+// to 1e24.
+GY_D int ray_exponent(V3 d) {
+    const float m = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
+    return (m >= 1e-24f && m <= kDirMin) || (m >= kDirMax && m <= 1e24f) ? -ilogbf(m) : 0;
+}
+// QUERY: the ray is a caller's, whose direction may have any length.
+template <bool ANY, int STACK, bool COUNT = false, bool SPH = false, bool QUERY = false>
 GY_D bool find_hit(const SceneDev& S, V3 o, V3 d, float tmin, float tmax, Hit* hit, uint32_t* stack, int stride,
                    uint32_t* n_node = nullptr, uint32_t* n_tri = nullptr) {
     uint32_t deep[STACK - kPathLds];
     Trav t;
-    trav_init(t, o, d, tmin, tmax);
+    const int k = QUERY ? ray_exponent(d) : 0;
+    if (k != 0) trav_init(t, o, v3(ldexpf(d.x, k), ldexpf(d.y, k), ldexpf(d.z, k)), ldexpf(tmin, -k), ldexpf(tmax, -k));
+    else trav_init(t, o, d, tmin, tmax);
     const int r = trav_run<ANY, kPathLds, COUNT>(S, t, stack, stride, SpillPrivate<STACK - kPathLds>{deep}, 0, n_node, n_tri);
+    if (k != 0) t.best = t.best_prim >= 0 ? ldexpf(t.best, k) : tmax;
     if (SPH && S.n_sph > 0) {
         const V3 inv = v3(1.f / d.x, 1.f / d.y, 1.f / d.z);
-        if (ANY) return r == 2 || sph_any(S, t.o, inv, tmin, tmax);
-        sph_closest(S, t.o, t.d, inv, tmin, tmax, &t.best, &t.best_prim, &t.bb1, &t.bb2);
+        if (ANY) return r == 2 || sph_any(S, o, inv, tmin, tmax);
+        sph_closest(S, o, d, inv, tmin, tmax, &t.best, &t.best_prim, &t.bb1, &t.bb2);
     }
     if (ANY) {
         if (r == 2) hit->prim = t.best_prim;

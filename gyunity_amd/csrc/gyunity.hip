@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(256) k_trace_closest(SceneDev S, const gy_ray*
     const float4 a = rp[0], b = rp[1];
     Hit h;
     gy_hit out;
-    if (find_hit<false, STACK, false, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256)) {
+    if (find_hit<false, STACK, false, SPH, true>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256)) {
         out.t = h.t;
         out.prim = h.prim;
         out.b1 = h.b1;
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256) k_trace_any(SceneDev S, const gy_ray* __r
     const float4* rp = reinterpret_cast<const float4*>(rays + i);
     const float4 a = rp[0], b = rp[1];
     Hit h;
-    occ[i] = find_hit<true, STACK, false, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256) ? 1 : 0;
+    occ[i] = find_hit<true, STACK, false, SPH, true>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256) ? 1 : 0;
 }
 
 __device__ inline void wave_add_u64(unsigned long long* dst, uint64_t v) {
@@ -195,7 +195,7 @@ __global__ void __launch_bounds__(256) k_count_visits(SceneDev S, const gy_ray* 
         const float4* rp = reinterpret_cast<const float4*>(rays + i);
         const float4 a = rp[0], b = rp[1];
         Hit h;
-        find_hit<false, STACK, true, SPH>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256, &nn, &nt);
+        find_hit<false, STACK, true, SPH, true>(S, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, &h, stack + threadIdx.x, 256, &nn, &nt);
     }
     wave_add_u64(&counters[0], nn);
     wave_add_u64(&counters[1], nt);

@@ -144,6 +144,29 @@ def test_hits_are_the_brute_force_hits(gpu_ctx, kind, n, leaf):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1e-9, 1.1e-10, 0.9e-10, 1e-12, 1e-20, 1e17, 0.9e18, 1.1e18, 1e20, 1e22])
+def test_short_and_long_directions_keep_the_culling(gpu_ctx, scale):
+    # directions beyond the slab test's reach of 1e-10 to 1e18: the hits of the
+    # brute force, and no more nodes than for directions of length 1
+    rng = np.random.default_rng(5)
+    tri = soup("random", 900, rng)
+    rays = rays_for(tri, 3000, rng)
+    rays["dir"] /= np.abs(rays["dir"]).max(1, keepdims=True)
+    scaled = rays.copy()
+    with np.errstate(under="ignore"):
+        scaled["dir"] = rays["dir"] * np.float32(scale)
+        scaled["tmax"] = rays["tmax"] / np.float32(scale)
+    t, prim, b1, b2, occluded = (np.concatenate(p) for p in zip(*(brute_force(tri, r) for r in np.array_split(scaled, 20))))
+    assert 0.2 < occluded.mean()
+    with g.Scene(gpu_ctx, scene(tri)) as sc:
+        hits, any_hit = sc.trace_closest(scaled), sc.trace_any(scaled)
+        visits, plain = sc.count_visits(scaled), sc.count_visits(rays)
+    assert np.array_equal(hits["prim"], prim) and np.array_equal(hits["t"], t)
+    assert np.array_equal(hits["b1"], b1) and np.array_equal(hits["b2"], b2) and np.array_equal(any_hit, occluded)
+    assert visits[0] < 1.05 * plain[0] and visits[1] < 1.05 * plain[1]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind,n", [("chain", 150), ("overlap", 20000)])
 def test_deep_stacks_render_alike_in_both_forms(gpu_ctx, kind, n):
     # the stack's deep entries go to global memory in the wavefront's trace
