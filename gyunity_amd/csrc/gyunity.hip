@@ -201,10 +201,8 @@ __global__ void __launch_bounds__(256) k_count_visits(SceneDev S, const gy_ray* 
     wave_add_u64(&counters[1], nt);
 }
 
-// WAVES per SIMD: five (96 VGPRs, some spilled) for launches that fill the card,
-// 16.1 ms for 3.3M paths of depth 10 over 82k triangles against 16.6 at four,
-// 18.0 at three and 24.0 without the hint; three (no spills in the loop, which
-// wait on scratch memory) for launches that do not (kMegaSmallWaves).
+// WAVES per SIMD: five (96 VGPRs, some spilled), four or three, by the size of
+// the tree and of the launch (LaunchMegaFilm).
 template <int STACK, int BLOCK, bool ENV, bool SPH, int WAVES = 5>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES)))
 k_pt_megakernel(SceneDev S, PathParams P, FilmDev F, int s0, int n_s,
@@ -754,13 +752,36 @@ int LaunchMegaT(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, i
     return CheckLaunch(c, "k_pt_megakernel");
 }
 
+template <int STACK, int WAVES>
+int LaunchMegaBlock(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, int s0, int n_s, int block, bool count, bool timed) {
+    if (block == 64) return LaunchMegaT<STACK, 64, false, WAVES>(c, sc, film, P, s0, n_s, count, timed);
+    if constexpr (STACK == kStackSmall)
+        if (block == 256) return LaunchMegaT<STACK, 256, false, WAVES>(c, sc, film, P, s0, n_s, count, timed);
+    return LaunchMegaT<STACK, 128, false, WAVES>(c, sc, film, P, s0, n_s, count, timed);
+}
+
 // The megakernel over one pass into `film` (the scene's own film, or the
 // no-alloc entry point's).  Scenes with spheres run the sphere instantiation
-// at 128 threads a block.  block 0 is automatic: 128 threads, or one wave a
-// block of the three-wave instantiation when the pass has no more waves than
-// that keeps resident; such a launch is a chain of latencies, and its waves
-// spread over twice the CUs (16,384 paths of depth 5: 197 -> 160 us).
+// at 128 threads a block.
+//
+// block 0 is automatic: 128 threads, or one wave a block of the three-wave
+// instantiation when the pass has no more waves than that keeps resident; such
+// a launch is a chain of latencies, spilled registers are on it, and its waves
+// spread over twice the CUs.  64 to 3072 waves of depth 6, against five waves a
+// SIMD and 128 threads: Cornell room 0.32 -> 0.30 ms at 256 waves, 0.39 -> 0.32
+// at 1024, 0.58 -> 0.42 at 3072; 1.31M triangles 1.01 -> 0.92, 1.07 -> 0.99,
+// 1.31 -> 1.15; 5,132 and 82k triangles between those.
+//
+// Larger launches: a tree whose records lie in one XCD's L2 (kTreeL2) misses
+// little and would rather have its registers than a fifth wave to hide misses
+// behind.  701 x 523, 9 samples, depth 10, five waves against four: Cornell room
+// 6.5 -> 5.5 ms, 1,292 triangles 10.1 -> 9.4, 5,132 10.6 -> 10.1; beyond it 82k
+// triangles 12.0 -> 12.2 and 1.31M 13.6 -> 14.1.  Three waves win only in the
+// Cornell room (5.0) and lose 3% to the rough dielectric at 5,132 triangles.
+// Trees deep enough for the large stack take three, with its private part in
+// mind: 300 nested triangles, 256 x 256, 8 samples 0.51 -> 0.45 ms.
 constexpr int kMegaSmallWaves = 3;
+constexpr int64_t kTreeL2 = 4 << 20;
 int LaunchMegaFilm(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, int s0, int n_s, int block, bool count,
                    bool timed) {
     if (sc->dev.n_sph > 0)
@@ -772,13 +793,12 @@ int LaunchMegaFilm(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P
             return sc->stack <= 64 ? LaunchMegaT<64, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed)
                                    : LaunchMegaT<192, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed);
     }
-    if (sc->stack <= 64) {
-        if (block == 64) return LaunchMegaT<64, 64, false>(c, sc, film, P, s0, n_s, count, timed);
-        if (block == 256) return LaunchMegaT<64, 256, false>(c, sc, film, P, s0, n_s, count, timed);
-        return LaunchMegaT<64, 128, false>(c, sc, film, P, s0, n_s, count, timed);
-    }
-    if (block == 64) return LaunchMegaT<192, 64, false>(c, sc, film, P, s0, n_s, count, timed);
-    return LaunchMegaT<192, 128, false>(c, sc, film, P, s0, n_s, count, timed);
+    const bool in_l2 = sc->dev.n_nodes * (int64_t)sizeof(WideNode) + sc->dev.n_tri * (int64_t)48 <= kTreeL2;
+    if (sc->stack == kStackSmall)
+        return in_l2 ? LaunchMegaBlock<kStackSmall, 4>(c, sc, film, P, s0, n_s, block, count, timed)
+                     : LaunchMegaBlock<kStackSmall, 5>(c, sc, film, P, s0, n_s, block, count, timed);
+    return in_l2 ? LaunchMegaBlock<kStackLarge, 3>(c, sc, film, P, s0, n_s, block, count, timed)
+                 : LaunchMegaBlock<kStackLarge, 5>(c, sc, film, P, s0, n_s, block, count, timed);
 }
 
 int LaunchMega(Ctx* c, Scene* sc, const PathParams& P, int s0, int n_s, int block, bool count) {

@@ -184,6 +184,26 @@ def test_deep_stacks_render_alike_in_both_forms(gpu_ctx, kind, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("spp", [48, 49])  # 64 x 64: 3072 waves, the most of a small launch at 256 CUs, and 3136
+@pytest.mark.parametrize("kind,n", [("random", 300), ("ico", 6), ("chain", 300)])  # tree within an L2, beyond it, deep
+def test_megakernel_forms_render_alike(gpu_ctx, kind, n, spp):
+    # every instantiation that the sizes of the launch and of the tree choose
+    # between, and the explicit block sizes: the wavefront's film
+    if kind == "ico":
+        sa, _, _ = g.generate_scene(g.GY_SCENE_ICOSPHERE_GGX, 1, n)
+        cam = g.camera((0.5, 0.5, 2.35), (0.5, 0.5, 0.0), (0, 1, 0), 40.0, 64, 64)
+    else:
+        sa = scene(soup(kind, n, np.random.default_rng(n)), lights=n // 2)
+        cam = g.camera((1.0, 1.0, 4.0), (0.6, 0.6, 0.0), (0, 1, 0), 50.0, 64, 64)
+    with g.Scene(gpu_ctx, sa, max_leaf_size=1) as sc:
+        want = sc.render(cam, g.render_params(spp, 3, mode=g.GY_RENDER_WAVEFRONT))
+        assert want[0].sum() > 0
+        for block in (0, 64, 128, 256):
+            got = sc.render(cam, g.render_params(spp, 3, mode=g.GY_RENDER_MEGAKERNEL, block_size=block))
+            assert np.array_equal(got[0], want[0], equal_nan=True) and np.array_equal(got[1], want[1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind,n", [("random", 64), ("random", 3000), ("chain", 150), ("wall", 300)])
 def test_both_builders_trees_give_the_same_hits(gpu_ctx, kind, n):
     # the device collapses its own binary trees of more than 1024 nodes, the
