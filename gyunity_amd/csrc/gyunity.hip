@@ -265,9 +265,10 @@ __global__ void __launch_bounds__(128) k_li_samples(SceneDev S, PathParams P, in
 }
 
 // LightTracing: one light path per thread, sample index = thread index.
-// Five waves per SIMD (136 VGPRs and three without the hint): 9% faster.
-template <int STACK, int BLOCK, bool ENV>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) k_lt(SceneDev S, PathParams P, LightCamDev C, int64_t n, float total,
+// WAVES per SIMD: five (136 VGPRs and three without the hint: 9% slower), or
+// four over trees that an L1 holds (LtKernelOf).
+template <int STACK, int BLOCK, bool ENV, int WAVES>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) k_lt(SceneDev S, PathParams P, LightCamDev C, int64_t n, float total,
                                               float* __restrict__ splat) {
     __shared__ uint32_t stack[kPathLds * BLOCK];
     const int64_t t = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
@@ -752,6 +753,9 @@ int LaunchMegaT(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, i
     return CheckLaunch(c, "k_pt_megakernel");
 }
 
+// What a traversal reads: nodes and the triangles' intersection records.
+int64_t TreeBytes(const Scene* sc) { return sc->dev.n_nodes * (int64_t)sizeof(WideNode) + sc->dev.n_tri * (int64_t)48; }
+
 template <int STACK, int WAVES>
 int LaunchMegaBlock(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, int s0, int n_s, int block, bool count, bool timed) {
     if (block == 64) return LaunchMegaT<STACK, 64, false, WAVES>(c, sc, film, P, s0, n_s, count, timed);
@@ -793,7 +797,7 @@ int LaunchMegaFilm(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P
             return sc->stack <= 64 ? LaunchMegaT<64, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed)
                                    : LaunchMegaT<192, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed);
     }
-    const bool in_l2 = sc->dev.n_nodes * (int64_t)sizeof(WideNode) + sc->dev.n_tri * (int64_t)48 <= kTreeL2;
+    const bool in_l2 = TreeBytes(sc) <= kTreeL2;
     if (sc->stack == kStackSmall)
         return in_l2 ? LaunchMegaBlock<kStackSmall, 4>(c, sc, film, P, s0, n_s, block, count, timed)
                      : LaunchMegaBlock<kStackSmall, 5>(c, sc, film, P, s0, n_s, block, count, timed);
@@ -1129,7 +1133,27 @@ extern "C" int gy_scene_set_environment(gy_scene* s, const float* rgb, int32_t w
 
 namespace gy {
 int LightTracingWavefront(Ctx* c, Scene* sc, const PathParams& P, const LightCamDev& C, int64_t n, float total, float* splat);
+
+// Four waves a SIMD where the tree's records lie in the 32 KB L1: 512 x 512, 16
+// samples, depth 6 in the Cornell room 3.38 -> 3.22 ms (its splats' atomics
+// collide less).  Beyond it four waves hide too little: 23 KB of tree 5.59 ->
+// 5.66, 82k triangles 8.5 -> 9.0.
+using LtKernel = void (*)(SceneDev, PathParams, LightCamDev, int64_t, float, float*);
+template <int STACK, bool ENV, int WAVES>
+LtKernel LtKernelBlock(int block) {
+    return block == 64 ? k_lt<STACK, 64, ENV, WAVES> : block == 256 ? k_lt<STACK, 256, ENV, WAVES> : k_lt<STACK, 128, ENV, WAVES>;
 }
+template <int STACK, int WAVES>
+LtKernel LtKernelEnv(bool env, int block) {
+    return env ? LtKernelBlock<STACK, true, WAVES>(block) : LtKernelBlock<STACK, false, WAVES>(block);
+}
+constexpr int64_t kTreeL1 = 32 << 10;
+static LtKernel LtKernelOf(const Scene* sc, int block) {
+    const bool env = sc->dev.env.w > 0, in_l1 = TreeBytes(sc) <= kTreeL1;
+    if (sc->stack == kStackSmall) return in_l1 ? LtKernelEnv<kStackSmall, 4>(env, block) : LtKernelEnv<kStackSmall, 5>(env, block);
+    return in_l1 ? LtKernelEnv<kStackLarge, 4>(env, block) : LtKernelEnv<kStackLarge, 5>(env, block);
+}
+}  // namespace gy
 
 // LightTracing::Render (integrator/LT.h:17-53): spp light paths per pixel
 // index, rgb gets the film's splat sums (W x H x 3; the film has no samples,
@@ -1178,14 +1202,7 @@ extern "C" int gy_render_light_tracing(gy_scene* s, const gy_camera_desc* cam, c
         // 1.31M-triangle workload (86.6 Mpaths/s against 84.1 at 128, 81.4 at 256)
         const int bs = (p->block_size == 128 || p->block_size == 256) ? p->block_size : 64;
         const unsigned blocks = (unsigned)((n + bs - 1) / bs);
-        void (*kern)(SceneDev, PathParams, LightCamDev, int64_t, float, float*);
-        if (sc->dev.env.w > 0)
-            kern = sc->stack <= 64 ? (bs == 64 ? k_lt<64, 64, true> : bs == 256 ? k_lt<64, 256, true> : k_lt<64, 128, true>)
-                                   : (bs == 64 ? k_lt<192, 64, true> : bs == 256 ? k_lt<192, 256, true> : k_lt<192, 128, true>);
-        else
-            kern = sc->stack <= 64 ? (bs == 64 ? k_lt<64, 64, false> : bs == 256 ? k_lt<64, 256, false> : k_lt<64, 128, false>)
-                                   : (bs == 64 ? k_lt<192, 64, false> : bs == 256 ? k_lt<192, 256, false> : k_lt<192, 128, false>);
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(bs), 0, c->stream, sc->dev, P, C, n, (float)n, (float*)d);
+        hipLaunchKernelGGL(LtKernelOf(sc, bs), dim3(blocks), dim3(bs), 0, c->stream, sc->dev, P, C, n, (float)n, (float*)d);
         rc = CheckLaunch(c, "k_lt");
     }
     if (rc == GY_OK) {

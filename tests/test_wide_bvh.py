@@ -204,6 +204,21 @@ def test_megakernel_forms_render_alike(gpu_ctx, kind, n, spp):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,n", [("random", 64), ("random", 3000), ("chain", 150)])  # tree within the L1 or beyond
+def test_light_tracing_forms_splat_alike(gpu_ctx, kind, n):
+    # both forms add the same splats in another order: at most 64 * 40 * 8 * 4
+    # FP32 additions of one sign in a pixel
+    sa = scene(soup(kind, n, np.random.default_rng(n)), lights=n // 2)
+    cam = g.camera((1.0, 1.0, 4.0), (0.6, 0.6, 0.0), (0, 1, 0), 50.0, 64, 40)
+    with g.Scene(gpu_ctx, sa, max_leaf_size=1) as sc:
+        want = sc.render_light_tracing(cam, g.render_params(8, 4, mode=g.GY_RENDER_WAVEFRONT))
+        assert want.sum() > 0
+        for block in (0, 64, 128, 256):
+            got = sc.render_light_tracing(cam, g.render_params(8, 4, mode=g.GY_RENDER_MEGAKERNEL, block_size=block))
+            assert np.allclose(got, want, rtol=81920 * 2.0 ** -24, atol=0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind,n", [("random", 64), ("random", 3000), ("chain", 150), ("wall", 300)])
 def test_both_builders_trees_give_the_same_hits(gpu_ctx, kind, n):
     # the device collapses its own binary trees of more than 1024 nodes, the
