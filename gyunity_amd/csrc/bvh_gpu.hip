@@ -534,54 +534,93 @@ __global__ void k_bvh_small(BuildDev B, uint32_t* idx, uint32_t nsmall) {
 }
 
 // ---------------------------------------------------------------- wide tree
+// The traversal tree: compressed wide nodes (byte boxes on a grid of the node's
+// own) after Ylitie, Karras and Laine, "Efficient incoherent ray traversal on
+// GPUs through compressed wide BVHs", 2017, here four wide and collapsed from
+// the binary tree by surface area as in Wald, Benthin and Boulos, "Getting rid
+// of packets", 2008.
+//
 // The children of the wide node that stands for binary node `open`: that
 // node's, and while there is room the interior child with the largest surface
 // area gives way to its own two children (large boxes are entered most often,
-// so opening them saves the most node visits).
+// so opening them saves the most node visits).  Axes outermost, so that the
+// four children's values are one vector on the host and none is indexed at run
+// time on the device (kid_set), where that would go through scratch memory.
 struct WideKids {
-    float box[4][6];
+    float lo[3][4], hi[3][4];
+    float area[4];            // -1: not an interior child
     uint32_t ref[4], cnt[4];  // as in the binary node: count 0 for an interior child
     int n;
     uint32_t inner;  // interior children
 };
+template <class T>
+__host__ __device__ inline void kid_set(T (&a)[4], int s, T v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = i == s ? v : a[i];
+}
 __host__ __device__ inline float bits_float(uint32_t v) { return __builtin_bit_cast(float, v); }
+__host__ __device__ inline float lesser(float a, float b) { return a < b ? a : b; }
+__host__ __device__ inline float greater(float a, float b) { return a > b ? a : b; }
 // pad: added to every side of the boxes.
 __host__ __device__ inline WideKids wide_open(const uint4* binary, uint32_t open, float pad) {
     WideKids w;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            w.lo[k][s] = __builtin_huge_valf();
+            w.hi[k][s] = -__builtin_huge_valf();
+        }
+        w.area[s] = -1.f;
+        w.ref[s] = w.cnt[s] = 0u;
+    }
     int n = 0, at = 0;
+    uint32_t inner = 0;
     while (true) {
         const uint4* b = binary + (size_t)open * 4;
         const uint4 q0 = b[0], q1 = b[1], q2 = b[2], q3 = b[3];
-        const uint32_t q[16] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+        const float box[2][6] = {{bits_float(q0.x), bits_float(q0.y), bits_float(q0.z), bits_float(q0.w), bits_float(q1.x), bits_float(q1.y)},
+                                 {bits_float(q1.z), bits_float(q1.w), bits_float(q2.x), bits_float(q2.y), bits_float(q2.z), bits_float(q2.w)}};
+        const uint32_t ref[2] = {q3.x, q3.y}, cnt[2] = {q3.z, q3.w};
         bool first = true;  // the first child takes the opened child's place
+#pragma unroll
         for (int c = 0; c < 2; ++c) {
-            if (q[12 + c] == kEmptyRef) continue;
+            if (ref[c] == kEmptyRef) continue;
             const int s = first ? at : n;
             if (s == n) ++n;
             first = false;
+            float e[3];
+#pragma unroll
             for (int k = 0; k < 3; ++k) {
-                w.box[s][k] = bits_float(q[6 * c + k]) - pad;
-                w.box[s][3 + k] = bits_float(q[6 * c + 3 + k]) + pad;
+                const float l = box[c][k] - pad, h = box[c][3 + k] + pad;
+                kid_set(w.lo[k], s, l);
+                kid_set(w.hi[k], s, h);
+                e[k] = h - l;
             }
-            w.ref[s] = q[12 + c];
-            w.cnt[s] = q[14 + c];
+            kid_set(w.ref, s, ref[c]);
+            kid_set(w.cnt, s, cnt[c]);
+            const float area = e[0] * e[1] + e[1] * e[2] + e[2] * e[0];
+            // an infinite box (or one whose area is not a number) is opened like any other
+            kid_set(w.area, s, cnt[c] != 0u ? -1.f : (area >= 0.f ? area : __builtin_huge_valf()));
+            inner += cnt[c] == 0u ? 1u : 0u;
         }
+        if (n == 4) break;
         at = -1;
         float big = -1.f;
-        for (int s = 0; s < n && n < 4; ++s) {
-            const float x = w.box[s][3] - w.box[s][0], y = w.box[s][4] - w.box[s][1], z = w.box[s][5] - w.box[s][2];
-            const float area = x * y + y * z + z * x;
-            if (w.cnt[s] == 0 && !(area <= big)) {
-                big = area;
+        uint32_t next = 0;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (w.area[s] > big) {
+                big = w.area[s];
                 at = s;
+                next = w.ref[s];
             }
-        }
         if (at < 0) break;
-        open = w.ref[at];
+        open = next;
+        --inner;
     }
     w.n = n;
-    w.inner = 0;
-    for (int s = 0; s < n; ++s) w.inner += w.cnt[s] == 0 ? 1u : 0u;
+    w.inner = inner;
     return w;
 }
 // The node with those children, the interior ones at `next` and on.
@@ -589,37 +628,43 @@ __host__ __device__ inline gyd::WideNode wide_make(const WideKids& w, uint32_t n
     // the children's grid: 255 steps an axis, the node's box between steps 2
     // and 252 (FP32 places the origin within two steps, since a padded box is
     // at least 60 ulp wide); bytes are rounded outward with 1/128 step to spare
-    // for the traversal's FP32 distances
+    // for the traversal's FP32 distances, and 0.0079 - 1/128 for the rounding
+    // of the steps themselves (four roundings of values up to 253: 6.1e-5)
     gyd::WideNode o;
-    for (int k = 0; k < 6; ++k) o.q[k] = 0u;
+#pragma unroll
     for (int k = 0; k < 3; ++k) {
-        float lo = __builtin_huge_valf(), hi = -__builtin_huge_valf();
-        for (int s = 0; s < w.n; ++s) {
-            lo = fminf(lo, w.box[s][k]);
-            hi = fmaxf(hi, w.box[s][3 + k]);
-        }
+        const float* L = w.lo[k];
+        const float* H = w.hi[k];
+        const float lo = lesser(lesser(L[0], L[1]), lesser(L[2], L[3])), hi = greater(greater(H[0], H[1]), greater(H[2], H[3]));
         // beyond 1e11 (or infinite, or NaN) a step times a ray's 1 / direction
         // can leave FP32's range; the axis then takes part in no decision: the
         // children's planes lie further out than any that FP32 can test
-        const bool open = !(hi - lo <= 1e11f);
-        const float step = open ? 1e30f : fmaxf((hi - lo) * (1.f / 250.f), 1e-30f);
-        o.org[k] = open ? -1.25e32f : lo - 2.f * step;
+        bool open = !(hi - lo <= 1e11f);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) open = open || (s < w.n && !(H[s] - L[s] <= 1e11f));
+        const float step = open ? 1e30f : greater((hi - lo) * (1.f / 250.f), 1e-30f);
+        const float org = open ? -1.25e32f : lo - 2.f * step;
+        o.org[k] = org;
         o.scale[k] = step * 16777216.f;
+        const float inv = 1.f / step;
+        uint32_t mn = 0, mx = 0;
+#pragma unroll
         for (int s = 0; s < 4; ++s) {
-            int mn = 255, mx = 0;  // absent: inverted
-            if (s < w.n && open) {
-                mn = 0;
-                mx = 255;
-            } else if (s < w.n) {
-                mn = (int)floor(((double)w.box[s][k] - (double)o.org[k]) / (double)step - 0.0078125);
-                mx = (int)ceil(((double)w.box[s][3 + k] - (double)o.org[k]) / (double)step + 0.0078125);
-                mn = mn < 0 ? 0 : (mn > 255 ? 255 : mn);
-                mx = mx < 0 ? 0 : (mx > 255 ? 255 : mx);
+            const float x = (L[s] - org) * inv - 0.0079f, y = (H[s] - org) * inv + 0.0079f;
+            // absent children: infinities the wrong way round, 255 and 0
+            int a = (int)lesser(greater(x, 0.f), 255.f), b = (int)lesser(greater(y, 0.f), 255.f);
+            b += (float)b < y && b < 255 ? 1 : 0;
+            if (open) {
+                a = s < w.n ? 0 : 255;
+                b = s < w.n ? 255 : 0;
             }
-            o.q[2 * k] |= (uint32_t)mn << (8 * s);
-            o.q[2 * k + 1] |= (uint32_t)mx << (8 * s);
+            mn |= (uint32_t)a << (8 * s);
+            mx |= (uint32_t)b << (8 * s);
         }
+        o.q[2 * k] = mn;
+        o.q[2 * k + 1] = mx;
     }
+#pragma unroll
     for (int s = 0; s < 4; ++s) {
         if (s >= w.n) o.entry[s] = gyd::kTravLeaf;  // an empty leaf
         else if (w.cnt[s] == 0) o.entry[s] = next++;
@@ -627,22 +672,54 @@ __host__ __device__ inline gyd::WideNode wide_make(const WideKids& w, uint32_t n
     }
     return o;
 }
+// Node w of the tree and its children's places in src; claim(k) gives the first
+// of k new nodes.
+template <class Claim>
+__host__ __device__ inline void wide_node(const uint4* binary, gyd::WideNode* wide, uint32_t* src, uint32_t w, float pad, const Claim& claim) {
+    const WideKids kids = wide_open(binary, src[w], pad);
+    uint32_t i = kids.inner ? claim(kids.inner) : 0u;
+    wide[w] = wide_make(kids, i);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+        if (s < kids.n && kids.cnt[s] == 0) src[i++] = kids.ref[s];
+}
 
-// One level of the wide tree: node w of the level stands for the binary node
-// src[w].  ctr: nodes so far, level begin, level end, levels.  The order of the
-// nodes of a level is not fixed; no result depends on it.  1.31M triangles:
-// 0.44M nodes from 1.31M.
+// The tree is collapsed level by level: node w stands for binary node src[w].
+// ctr: nodes so far, level begin, level end, levels.  The order of the nodes of
+// a level is not fixed; no result depends on it.
+//
+// One workgroup walks all levels of a tree of up to kWideBlock binary nodes: a
+// launch (and a wait between two) a level cost more than such a level's work.
+constexpr int64_t kWideBlock = 1 << 16;
+__global__ void __launch_bounds__(1024) k_wide_block(const uint4* __restrict__ binary, gyd::WideNode* __restrict__ wide, uint32_t* src,
+                                                     uint32_t* __restrict__ ctr, float pad) {
+    __shared__ uint32_t nodes;
+    if (threadIdx.x == 0) {
+        src[0] = 0u;
+        nodes = 1u;
+    }
+    __syncthreads();
+    uint32_t begin = 0, end = 1, levels = 0;
+    while (begin < end) {  // the same in every thread
+        for (uint32_t w = begin + threadIdx.x; w < end; w += 1024)
+            wide_node(binary, wide, src, w, pad, [&](uint32_t k) { return atomicAdd(&nodes, k); });
+        __syncthreads();
+        begin = end;
+        end = nodes;
+        ++levels;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        ctr[0] = end;
+        ctr[1] = ctr[2] = end;
+        ctr[3] = levels;
+    }
+}
 __global__ void __launch_bounds__(64) k_wide_level(const uint4* __restrict__ binary, gyd::WideNode* __restrict__ wide,
                                                    uint32_t* __restrict__ src, uint32_t* __restrict__ ctr, float pad) {
     const uint32_t end = ctr[2];
-    for (uint32_t w = ctr[1] + blockIdx.x * 64 + threadIdx.x; w < end; w += gridDim.x * 64) {
-        const WideKids kids = wide_open(binary, src[w], pad);
-        const uint32_t next = kids.inner ? atomicAdd(&ctr[0], kids.inner) : 0u;
-        wide[w] = wide_make(kids, next);
-        uint32_t i = next;
-        for (int s = 0; s < kids.n; ++s)
-            if (kids.cnt[s] == 0) src[i++] = kids.ref[s];
-    }
+    for (uint32_t w = ctr[1] + blockIdx.x * 64 + threadIdx.x; w < end; w += gridDim.x * 64)
+        wide_node(binary, wide, src, w, pad, [&](uint32_t k) { return atomicAdd(&ctr[0], k); });
 }
 __global__ void k_wide_advance(uint32_t* ctr) {
     if (threadIdx.x != 0) return;
@@ -659,64 +736,101 @@ __global__ void k_wide_root(uint32_t* src, uint32_t* ctr) {
     ctr[3] = 0u;
 }
 
-constexpr uint32_t kWideHost = 1024;
-
-// The wide tree of the n binary nodes at `binary`, while they are still on the
-// device: built in `tmp` (room for n nodes) and `src` (n words), kept in an
-// allocation of its own size.  From the host's copy of the nodes it took their
-// upload (84 MB at 1.31M triangles) and four allocations more: 34 ms of a scene
-// creation that takes 120.
-int WideDevice(Ctx* c, const uint32_t* binary, int64_t n, int max_depth, float pad, void* tmp, uint32_t* src, uint32_t* ctr,
-               BVHBuild* out) {
-    const unsigned blocks = (unsigned)std::min<int64_t>((n + 63) / 64, 4096);
-    hipLaunchKernelGGL(k_wide_root, dim3(1), dim3(64), 0, c->stream, src, ctr);
-    for (int l = 0; l <= max_depth; ++l) {
-        hipLaunchKernelGGL(k_wide_level, dim3(blocks), dim3(64), 0, c->stream, (const uint4*)binary, (gyd::WideNode*)tmp, src, ctr, pad);
-        hipLaunchKernelGGL(k_wide_advance, dim3(1), dim3(64), 0, c->stream, ctr);
+// Queues the collapse of the n binary nodes at `binary` (max_depth levels), with
+// `src` (n words) and `ctr` (4 words) in b->scratch: a small tree goes straight
+// into an allocation of n nodes (a third to a half stays unused: at most 4 MB),
+// a large one into `tmp` (room for n nodes), from where BuildWide takes it.
+int WideLaunch(Ctx* c, const uint32_t* binary, int64_t n, int max_depth, float pad, void* tmp, uint32_t* src, uint32_t* ctr, BVHBuild* b) {
+    const uint4* bin = (const uint4*)binary;
+    b->wide_ctr = ctr;
+    if (n <= kWideBlock) {
+        const int rc = DevAlloc(c, &b->wide, (size_t)n * sizeof(gyd::WideNode));
+        if (rc != GY_OK) return rc;
+        hipLaunchKernelGGL(k_wide_block, dim3(1), dim3(1024), 0, c->stream, bin, (gyd::WideNode*)b->wide, src, ctr, pad);
+    } else {
+        b->wide_tmp = tmp;
+        const unsigned blocks = (unsigned)std::min<int64_t>((n + 63) / 64, 4096);
+        hipLaunchKernelGGL(k_wide_root, dim3(1), dim3(64), 0, c->stream, src, ctr);
+        for (int l = 0; l <= max_depth; ++l) {
+            hipLaunchKernelGGL(k_wide_level, dim3(blocks), dim3(64), 0, c->stream, bin, (gyd::WideNode*)tmp, src, ctr, pad);
+            hipLaunchKernelGGL(k_wide_advance, dim3(1), dim3(64), 0, c->stream, ctr);
+        }
     }
-    int rc = CheckLaunch(c, "wide bvh");
-    if (rc != GY_OK) return rc;
-    uint32_t h[4] = {0, 0, 0, 0};
-    hipError_t e = hipMemcpyAsync(h, ctr, 16, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) return HipFail(e, "wide bvh");
-    if (h[1] != h[2]) return Fail(GY_ERR_DEVICE, "wide bvh: levels left over");
-    rc = DevAlloc(c, &out->wide, (size_t)h[0] * sizeof(gyd::WideNode));
-    if (rc != GY_OK) return rc;
-    e = hipMemcpyAsync(out->wide, tmp, (size_t)h[0] * sizeof(gyd::WideNode), hipMemcpyDeviceToDevice, c->stream);
-    if (e != hipSuccess) {
-        DevFree(out->wide);
-        out->wide = nullptr;
-        return HipFail(e, "wide bvh copy");
-    }
-    out->n_wide = h[0];
-    out->wide_depth = (int32_t)h[3];
-    return GY_OK;
+    return CheckLaunch(c, "wide bvh");
 }
 
 }  // namespace
 
-// The wide tree of a binary tree on the host (padded boxes): the host's builds,
-// and the device's up to kWideHost nodes (a few tens of microseconds; the
-// device's launches and read-back take 0.2 ms).
-int BuildWideHost(Ctx* c, BVHBuild* b) {
-    std::vector<gyd::WideNode> out;
-    std::vector<uint32_t> src(1, 0u);
-    const uint4* binary = reinterpret_cast<const uint4*>(b->nodes.data());
-    size_t begin = 0;
-    b->wide_depth = 0;
-    while (begin < src.size()) {  // a level
-        const size_t end = src.size();
-        for (; begin < end; ++begin) {
-            const WideKids kids = wide_open(binary, src[begin], 0.f);
-            out.push_back(wide_make(kids, (uint32_t)src.size()));
-            for (int s = 0; s < kids.n; ++s)
-                if (kids.cnt[s] == 0) src.push_back(kids.ref[s]);
+// The traversal tree b->wide: what the device's build has under way, or that of
+// the host's binary tree (padded boxes), up to kWideHost nodes on the host and
+// larger ones on the device.  Scene creation with the two-wide tree, which was
+// uploaded as it is, and with this one, ms (triangles 1,292, 5,132, 20,492, 82k,
+// 1.31M): device's builds 1.96 1.92, 2.28 2.22, 3.29 3.14, 6.76 5.98, 126 123;
+// the host's 0.54 0.51, 2.05 2.08, 8.27 8.36, 34.4 34.3, 671 673.  A node costs
+// the host 80-200 ns (the tree of 1.31M triangles 110 ms), which kWideHost
+// bounds; the device takes 33 us for 1,285 binary nodes, 129 us for 20,481.
+constexpr int64_t kWideHost = 2048;
+int BuildWide(Ctx* c, BVHBuild* b) {
+    if (!b->scratch) {
+        const int64_t n = (int64_t)(b->nodes.size() / 16);
+        const size_t nodes = (size_t)n * sizeof(gyd::WideNode);
+        if (n <= kWideHost) {
+            std::vector<gyd::WideNode> out((size_t)n);
+            std::vector<uint32_t> src((size_t)n);
+            src[0] = 0u;
+            uint32_t begin = 0, end = 1;
+            b->wide_depth = 0;
+            while (begin < end) {  // a level
+                uint32_t next = end;
+                for (; begin < end; ++begin)
+                    wide_node(reinterpret_cast<const uint4*>(b->nodes.data()), out.data(), src.data(), begin, 0.f, [&](uint32_t k) {
+                        next += k;
+                        return next - k;
+                    });
+                end = next;
+                ++b->wide_depth;
+            }
+            b->n_wide = end;
+            return Upload(c, &b->wide, out.data(), (size_t)end * sizeof(gyd::WideNode));
         }
-        ++b->wide_depth;
+        // binary nodes, a large tree's wide nodes, src, counters
+        const size_t tmp = n > kWideBlock ? nodes : 0;
+        int rc = DevAlloc(c, &b->scratch, nodes + tmp + (size_t)n * 4 + 16);
+        if (rc != GY_OK) return rc;
+        char* base = (char*)b->scratch;
+        uint32_t* src = (uint32_t*)(base + nodes + tmp);
+        const hipError_t e = hipMemcpyAsync(base, b->nodes.data(), nodes, hipMemcpyHostToDevice, c->stream);
+        if (e != hipSuccess) return HipFail(e, "wide bvh upload");
+        rc = WideLaunch(c, (const uint32_t*)base, n, b->max_depth, 0.f, base + nodes, src, src + n, b);
+        if (rc != GY_OK) return rc;
     }
-    b->n_wide = (int64_t)out.size();
-    return Upload(c, &b->wide, out.data(), out.size() * sizeof(gyd::WideNode));
+    uint32_t h[4] = {0, 0, 0, 0};
+    hipError_t e = hipMemcpyAsync(h, b->wide_ctr, 16, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return HipFail(e, "wide bvh");
+    if (h[1] != h[2]) return Fail(GY_ERR_DEVICE, "wide bvh: levels left over");
+    if (b->wide_tmp) {
+        int rc = DevAlloc(c, &b->wide, (size_t)h[0] * sizeof(gyd::WideNode));
+        if (rc != GY_OK) return rc;
+        e = hipMemcpyAsync(b->wide, b->wide_tmp, (size_t)h[0] * sizeof(gyd::WideNode), hipMemcpyDeviceToDevice, c->stream);
+        // the copy is part of the build: traversal follows the tree's indices
+        // without bounds checks
+        rc = StreamSync(c, "wide bvh copy");
+        if (e != hipSuccess) rc = HipFail(e, "wide bvh copy");
+        if (rc != GY_OK) return rc;
+    }
+    b->n_wide = h[0];
+    b->wide_depth = (int32_t)h[3];
+    WideDrop(c, b);
+    return GY_OK;
+}
+
+// Ends the build on the device, whatever it came to; b->wide is the caller's.
+void WideDrop(Ctx* c, BVHBuild* b) {
+    if (!b->scratch) return;
+    (void)hipStreamSynchronize(c->stream);
+    DevFree(b->scratch);
+    b->scratch = nullptr;
 }
 
 // Build on the device, then copy nodes and leaf order back for the scene upload.
@@ -843,27 +957,24 @@ int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, float 
     const uint32_t nn = std::min(h[0], B.max_nodes);
     out->nodes.resize((size_t)nn * 16);
     out->tri_order.resize(n);
+    out->max_depth = (int32_t)h[3];
     e = hipMemcpyAsync(out->nodes.data(), B.nodes, (size_t)nn * 64, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out->tri_order.data(), B.idx[cur], n * 4, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return fail(e, "bvh download");
-    out->max_depth = (int32_t)h[3];
-    if (nn > kWideHost) {
-        // the triangles and their bounds (68 bytes each) are done with: a node
-        // takes 64, and there are fewer nodes than triangles
-        if ((size_t)nn * sizeof(gyd::WideNode) > o_idx0 - o_pos || (size_t)nn > (size_t)n) rc = Fail(GY_ERR_DEVICE, "wide bvh: more nodes than triangles");
-        else rc = WideDevice(c, B.nodes, nn, out->max_depth, pad, base + o_pos, (uint32_t*)B.tid[0], acc, out);
-        // the copy out of `base` is part of the build: traversal follows the
-        // tree's indices without bounds checks
-        const int sync = StreamSync(c, "wide bvh copy");
-        if (rc == GY_OK) rc = sync;
-        if (rc != GY_OK) {
-            DevFree(out->wide);
-            out->wide = nullptr;
-        }
+    // The traversal tree, in the space of the triangles and their bounds (68
+    // bytes each), which are done with: a node takes 64, and there are fewer
+    // nodes than triangles.  It is collapsed while the host prepares the
+    // scene's other arrays (BuildWide waits for it).
+    if ((size_t)nn * sizeof(gyd::WideNode) > o_idx0 - o_pos || (size_t)nn > (size_t)n) rc = Fail(GY_ERR_DEVICE, "wide bvh: more nodes than triangles");
+    else rc = WideLaunch(c, B.nodes, nn, out->max_depth, pad, base + o_pos, (uint32_t*)B.tid[0], acc, out);
+    out->scratch = base;
+    if (rc != GY_OK) {
+        WideDrop(c, out);
+        DevFree(out->wide);
+        out->wide = nullptr;
+        return rc;
     }
-    DevFree(base);
-    if (rc != GY_OK) return rc;
     out->n_leaves = h[4];
     out->max_leaf = max_leaf;
     out->sah_cost = BVHSahCost(*out);

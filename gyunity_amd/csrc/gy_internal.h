@@ -89,6 +89,9 @@ struct BVHBuild {
     double sah_cost = 0;
     // the traversal tree (gyd::WideNode records on the device), and its levels
     void* wide = nullptr;
+    // the build's device memory while that tree is under way; a large tree's
+    // nodes and its counters in it
+    void *scratch = nullptr, *wide_tmp = nullptr, *wide_ctr = nullptr;
     int64_t n_wide = 0;
     int32_t wide_depth = 0;
 };

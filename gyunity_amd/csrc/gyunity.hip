@@ -63,13 +63,17 @@ int DevAlloc(Ctx* c, void** p, size_t bytes) {
     return GY_OK;
 }
 
-int Upload(Ctx* c, void** p, const void* src, size_t bytes) {
+int UploadQueued(Ctx* c, void** p, const void* src, size_t bytes) {
     int rc = DevAlloc(c, p, bytes);
     if (rc != GY_OK) return rc;
     if (bytes == 0) return GY_OK;
     hipError_t e = hipMemcpyAsync(*p, src, bytes, hipMemcpyHostToDevice, c->stream);
-    if (e != hipSuccess) return HipFail(e, "hipMemcpyAsync H2D");
-    e = hipStreamSynchronize(c->stream);
+    return e == hipSuccess ? GY_OK : HipFail(e, "hipMemcpyAsync H2D");
+}
+int Upload(Ctx* c, void** p, const void* src, size_t bytes) {
+    int rc = UploadQueued(c, p, src, bytes);
+    if (rc != GY_OK || bytes == 0) return rc;
+    hipError_t e = hipStreamSynchronize(c->stream);
     return e == hipSuccess ? GY_OK : HipFail(e, "hipStreamSynchronize");
 }
 
@@ -342,17 +346,19 @@ static float LightCdf(const std::vector<float>& func, std::vector<float>* cdf) {
 }
 
 // The light table on the device: triangle (-1: the environment light), Le,
-// power CDF and function.  Replaces the previous table.
+// power CDF and function.  Replaces the previous table.  Without `wait` the
+// vectors have to stay until the stream is waited for.
 static int UploadLights(Ctx* c, Scene* sc, const std::vector<int32_t>& tri, const std::vector<float>& le,
-                        const std::vector<float>& func, const std::vector<float>& cdf) {
+                        const std::vector<float>& func, const std::vector<float>& cdf, bool wait = true) {
+    const auto upload = wait ? Upload : UploadQueued;
     void* bufs[4] = {nullptr, nullptr, nullptr, nullptr};
     const size_t n = tri.size();
     int rc = GY_OK;
     if (n > 0) {
-        if (rc == GY_OK) rc = Upload(c, &bufs[0], tri.data(), n * 4);
-        if (rc == GY_OK) rc = Upload(c, &bufs[1], le.data(), n * 12);
-        if (rc == GY_OK) rc = Upload(c, &bufs[2], cdf.data(), cdf.size() * 4);
-        if (rc == GY_OK) rc = Upload(c, &bufs[3], func.data(), func.size() * 4);
+        if (rc == GY_OK) rc = upload(c, &bufs[0], tri.data(), n * 4);
+        if (rc == GY_OK) rc = upload(c, &bufs[1], le.data(), n * 12);
+        if (rc == GY_OK) rc = upload(c, &bufs[2], cdf.data(), cdf.size() * 4);
+        if (rc == GY_OK) rc = upload(c, &bufs[3], func.data(), func.size() * 4);
     }
     if (rc != GY_OK) {
         for (void* b : bufs) DevFree(b);
@@ -501,6 +507,7 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     sc->stats.sah_cost = b.sah_cost;
     sc->d_nodes = b.wide;
     if (b.max_depth + 1 > 64) {
+        WideDrop(c, &b);
         SceneFree(sc);
         return Fail(GY_ERR_UNSUPPORTED, "BVH deeper than the 64-entry traversal stack");
     }
@@ -538,29 +545,37 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     for (int i = 0; i < d.n_tex; ++i)
         texinfo[i] = make_int4(d.tex_info[4 * i], d.tex_info[4 * i + 1], d.tex_info[4 * i + 2], d.tex_info[4 * i + 3]);
     void* p;
-    if ((rc = Upload(c, &p, tri.data(), tri.size() * sizeof(float4))) != GY_OK) goto fail;
+    if ((rc = UploadQueued(c, &p, tri.data(), tri.size() * sizeof(float4))) != GY_OK) goto fail;
     sc->d_tri = p;
     sc->dev.tri = (const float4*)p;
-    if ((rc = Upload(c, &p, shade.data(), shade.size() * sizeof(float4))) != GY_OK) goto fail;
+    if ((rc = UploadQueued(c, &p, shade.data(), shade.size() * sizeof(float4))) != GY_OK) goto fail;
     sc->d_shade = p;
     sc->dev.shade = (const float4*)p;
-    if (!b.wide && (rc = BuildWideHost(c, &b)) != GY_OK) goto fail;
+    rc = BuildWide(c, &b);
     sc->d_nodes = b.wide;
+    if (rc != GY_OK) goto fail;
     sc->dev.nodes = (const WideNode*)b.wide;
     sc->dev.n_nodes = (int32_t)b.n_wide;
     // the end mark, and at most three children of each node on a path
     sc->stack = 1 + 3 * b.wide_depth <= kStackSmall ? kStackSmall : kStackLarge;
-    if ((rc = Upload(c, &p, d.mats, (size_t)d.n_mat * GY_MAT_WORDS * 4)) != GY_OK) goto fail;
+    if ((rc = UploadQueued(c, &p, d.mats, (size_t)d.n_mat * GY_MAT_WORDS * 4)) != GY_OK) goto fail;
     sc->d_mats = p;
     sc->dev.mats = (const uint32_t*)p;
-    if ((rc = Upload(c, &p, texdata.data(), texdata.size() * 4)) != GY_OK) goto fail;
+    if ((rc = UploadQueued(c, &p, texdata.data(), texdata.size() * 4)) != GY_OK) goto fail;
     sc->d_tex = p;
     sc->dev.tex = (const float*)p;
     sc->tex_floats = (int64_t)texn;
-    if ((rc = Upload(c, &p, texinfo.data(), texinfo.size() * sizeof(int4))) != GY_OK) goto fail;
+    if ((rc = UploadQueued(c, &p, texinfo.data(), texinfo.size() * sizeof(int4))) != GY_OK) goto fail;
     sc->d_texinfo = p;
     sc->dev.tex_info = (const int4*)p;
-    if ((rc = UploadLights(c, sc, sc->area_tri, sc->area_le, func, cdf)) != GY_OK) goto fail;
+    if ((rc = UploadLights(c, sc, sc->area_tri, sc->area_le, func, cdf, false)) != GY_OK) goto fail;
+    // one wait for all copies: a wait each was half of the 0.14 ms that the
+    // Cornell room took
+    {
+        const hipError_t e = hipStreamSynchronize(c->stream);
+        if (e != hipSuccess) rc = HipFail(e, "scene upload");
+    }
+    if (rc != GY_OK) goto fail;
     sc->host_nodes = std::move(b.nodes);
     {
         auto t1 = std::chrono::steady_clock::now();
@@ -569,6 +584,8 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     *out = sc;
     return GY_OK;
 fail:
+    (void)hipStreamSynchronize(c->stream);  // copies under way read the locals above
+    WideDrop(c, &b);
     SceneFree(sc);
     return rc;
 }

@@ -113,6 +113,7 @@ struct Scene {
 int HipFail(hipError_t e, const char* what);
 int DevAlloc(Ctx* c, void** p, size_t bytes);
 int Upload(Ctx* c, void** p, const void* src, size_t bytes);
+int UploadQueued(Ctx* c, void** p, const void* src, size_t bytes);  // src stays as it is until the stream is waited for
 void DevFree(void* p);
 int Grow(Ctx* c, DevBuf* b, size_t bytes);
 int Fill32(Ctx* c, void* p, uint32_t v, int64_t n);
@@ -190,7 +191,9 @@ int BatchAdjoint(Ctx* c, Batch* b, const float* dimages, float* grad_tex, float*
 int BatchImages(Ctx* c, Batch* b, float* images);
 // GPU binned-SAH BVH build (bvh_gpu.hip).
 int BuildBVHDevice(Ctx* c, const float* pos, int32_t n_tri, int max_leaf, float pad, BVHBuild* out);
-// The wide tree of a binary tree on the host (padded boxes) into b->wide.
-int BuildWideHost(Ctx* c, BVHBuild* b);
+// The traversal tree into b->wide; WideDrop ends what a build that is given up
+// has under way.
+int BuildWide(Ctx* c, BVHBuild* b);
+void WideDrop(Ctx* c, BVHBuild* b);
 
 }  // namespace gy
