@@ -361,7 +361,7 @@ static int AdjointDevice(Scene* sc, const gy_camera_desc* cam, const gy_render_p
     if (sc->tex_floats == 0) return Fail(GY_ERR_INVALID, "gy_adjoint: the scene has no textures");
     if (sc->dev.env.w > 0) return Fail(GY_ERR_UNSUPPORTED, "gy_adjoint: scenes with an environment light");
     if (sc->dev.n_sph > 0) return Fail(GY_ERR_UNSUPPORTED, "gy_adjoint: scenes with spheres");
-    if (sc->stats.max_depth + 1 > 64) return Fail(GY_ERR_UNSUPPORTED, "gy_adjoint: BVH deeper than the traversal stack");
+    if (sc->stats.max_depth + 1 > kTreeLevels) return Fail(GY_ERR_UNSUPPORTED, "gy_adjoint: BVH deeper than the traversal stack");
     PathParams P;
     rc = MakePathParams(c, sc, *cam, *p, &P);
     if (rc != GY_OK) return rc;
@@ -378,12 +378,12 @@ static int AdjointDevice(Scene* sc, const gy_camera_desc* cam, const gy_render_p
         const int64_t threads = (int64_t)tilesX * tilesY * 64 * n_s;
         const unsigned blocks = (unsigned)((threads + kBlock - 1) / kBlock);
         const Grad G{grad, gle};
-        if (sc->stack <= 64) {
-            if (stored) hipLaunchKernelGGL((k_pt_adjoint<64, kBlock, true>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev, P, F, dI, G, s0, n_s);
-            else hipLaunchKernelGGL((k_pt_adjoint<64, kBlock, false>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev, P, F, dI, G, s0, n_s);
+        if (sc->stack == kStackSmall) {
+            if (stored) hipLaunchKernelGGL((k_pt_adjoint<kStackSmall, kBlock, true>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev, P, F, dI, G, s0, n_s);
+            else hipLaunchKernelGGL((k_pt_adjoint<kStackSmall, kBlock, false>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev, P, F, dI, G, s0, n_s);
         } else {
-            if (stored) hipLaunchKernelGGL((k_pt_adjoint<192, kBlock, true>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev, P, F, dI, G, s0, n_s);
-            else hipLaunchKernelGGL((k_pt_adjoint<192, kBlock, false>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev, P, F, dI, G, s0, n_s);
+            if (stored) hipLaunchKernelGGL((k_pt_adjoint<kStackLarge, kBlock, true>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev, P, F, dI, G, s0, n_s);
+            else hipLaunchKernelGGL((k_pt_adjoint<kStackLarge, kBlock, false>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev, P, F, dI, G, s0, n_s);
         }
         rc = CheckLaunch(c, "k_pt_adjoint");
     }
@@ -401,7 +401,7 @@ int BatchAdjoint(Ctx* c, Batch* b, const float* dI, float* grad, float* gle) {
     }
     if (sc->tex_floats == 0) return Fail(GY_ERR_INVALID, "gy_batch_adjoint: the scene has no textures");
     if (sc->dev.env.w > 0) return Fail(GY_ERR_UNSUPPORTED, "gy_batch_adjoint: scenes with an environment light");
-    if (sc->stats.max_depth + 1 > 64) return Fail(GY_ERR_UNSUPPORTED, "gy_batch_adjoint: BVH deeper than the traversal stack");
+    if (sc->stats.max_depth + 1 > kTreeLevels) return Fail(GY_ERR_UNSUPPORTED, "gy_batch_adjoint: BVH deeper than the traversal stack");
     constexpr int kBlock = kBatchAdjointBlock;
     const Grad G{grad, gle};
     // launches of at most 2^23 workgroups (2^30 samples)
@@ -410,11 +410,11 @@ int BatchAdjoint(Ctx* c, Batch* b, const float* dI, float* grad, float* gle) {
     TimerBegin(c, kKernOther);
     for (int64_t base = 0; base < b->adj_blocks && rc == GY_OK; base += kChunk) {
         const unsigned blocks = (unsigned)std::min(kChunk, b->adj_blocks - base);
-        if (sc->stack <= 64)
-            hipLaunchKernelGGL((k_batch_adjoint<64, kBlock>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev,
+        if (sc->stack == kStackSmall)
+            hipLaunchKernelGGL((k_batch_adjoint<kStackSmall, kBlock>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev,
                                (const BatchEntryDev*)b->table, (int32_t)b->entries.size(), dI, G, base);
         else
-            hipLaunchKernelGGL((k_batch_adjoint<192, kBlock>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev,
+            hipLaunchKernelGGL((k_batch_adjoint<kStackLarge, kBlock>), dim3(blocks), dim3(kBlock), 0, c->stream, sc->dev,
                                (const BatchEntryDev*)b->table, (int32_t)b->entries.size(), dI, G, base);
         rc = CheckLaunch(c, "k_batch_adjoint");
     }

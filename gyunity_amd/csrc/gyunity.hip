@@ -310,16 +310,16 @@ int LaunchTraceAnyT(Ctx* c, const SceneDev& S, const gy_ray* rays, int64_t n, in
 int LaunchTraceClosest(Ctx* c, Scene* sc, const gy_ray* rays, int64_t n, gy_hit* hits) {
     if (n <= 0) return GY_OK;
     if (sc->dev.n_sph > 0)
-        return sc->stack <= 64 ? LaunchTraceClosestT<64, true>(c, sc->dev, rays, n, hits)
-                               : LaunchTraceClosestT<192, true>(c, sc->dev, rays, n, hits);
-    return sc->stack <= 64 ? LaunchTraceClosestT<64, false>(c, sc->dev, rays, n, hits)
-                           : LaunchTraceClosestT<192, false>(c, sc->dev, rays, n, hits);
+        return sc->stack == kStackSmall ? LaunchTraceClosestT<kStackSmall, true>(c, sc->dev, rays, n, hits)
+                               : LaunchTraceClosestT<kStackLarge, true>(c, sc->dev, rays, n, hits);
+    return sc->stack == kStackSmall ? LaunchTraceClosestT<kStackSmall, false>(c, sc->dev, rays, n, hits)
+                           : LaunchTraceClosestT<kStackLarge, false>(c, sc->dev, rays, n, hits);
 }
 int LaunchTraceAny(Ctx* c, Scene* sc, const gy_ray* rays, int64_t n, int32_t* occ) {
     if (n <= 0) return GY_OK;
     if (sc->dev.n_sph > 0)
-        return sc->stack <= 64 ? LaunchTraceAnyT<64, true>(c, sc->dev, rays, n, occ) : LaunchTraceAnyT<192, true>(c, sc->dev, rays, n, occ);
-    return sc->stack <= 64 ? LaunchTraceAnyT<64, false>(c, sc->dev, rays, n, occ) : LaunchTraceAnyT<192, false>(c, sc->dev, rays, n, occ);
+        return sc->stack == kStackSmall ? LaunchTraceAnyT<kStackSmall, true>(c, sc->dev, rays, n, occ) : LaunchTraceAnyT<kStackLarge, true>(c, sc->dev, rays, n, occ);
+    return sc->stack == kStackSmall ? LaunchTraceAnyT<kStackSmall, false>(c, sc->dev, rays, n, occ) : LaunchTraceAnyT<kStackLarge, false>(c, sc->dev, rays, n, occ);
 }
 
 // ------------------------------------------------------------------ scene upload
@@ -506,10 +506,10 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     sc->stats.max_leaf_size = b.max_leaf;
     sc->stats.sah_cost = b.sah_cost;
     sc->d_nodes = b.wide;
-    if (b.max_depth + 1 > 64) {
+    if (b.max_depth + 1 > kTreeLevels) {
         WideDrop(c, &b);
         SceneFree(sc);
-        return Fail(GY_ERR_UNSUPPORTED, "BVH deeper than the 64-entry traversal stack");
+        return Fail(GY_ERR_UNSUPPORTED, "BVH of more than 64 levels (the traversal stack)");
     }
     for (size_t nidx = 0; nidx < b.nodes.size() / 16; ++nidx) {
         uint32_t* nd = &b.nodes[nidx * 16];
@@ -556,8 +556,8 @@ int SceneUpload(Ctx* c, const gy_scene_desc& d, const gy_bvh_params* bp, Scene**
     if (rc != GY_OK) goto fail;
     sc->dev.nodes = (const WideNode*)b.wide;
     sc->dev.n_nodes = (int32_t)b.n_wide;
-    // the end mark, and at most three children of each node on a path
-    sc->stack = 1 + 3 * b.wide_depth <= kStackSmall ? kStackSmall : kStackLarge;
+    // at most three children of each node on a path wait
+    sc->stack = 3 * b.wide_depth <= kStackSmall ? kStackSmall : kStackLarge;
     if ((rc = UploadQueued(c, &p, d.mats, (size_t)d.n_mat * GY_MAT_WORDS * 4)) != GY_OK) goto fail;
     sc->d_mats = p;
     sc->dev.mats = (const uint32_t*)p;
@@ -806,13 +806,13 @@ constexpr int64_t kTreeL2 = 4 << 20;
 int LaunchMegaFilm(Ctx* c, Scene* sc, const FilmState& film, const PathParams& P, int s0, int n_s, int block, bool count,
                    bool timed) {
     if (sc->dev.n_sph > 0)
-        return sc->stack <= 64 ? LaunchMegaT<64, 128, true>(c, sc, film, P, s0, n_s, count, timed)
-                               : LaunchMegaT<192, 128, true>(c, sc, film, P, s0, n_s, count, timed);
+        return sc->stack == kStackSmall ? LaunchMegaT<kStackSmall, 128, true>(c, sc, film, P, s0, n_s, count, timed)
+                               : LaunchMegaT<kStackLarge, 128, true>(c, sc, film, P, s0, n_s, count, timed);
     if (block == 0) {
         const int64_t waves = (int64_t)((film.width + 7) >> 3) * ((film.height + 7) >> 3) * n_s;
         if (!count && waves <= (int64_t)c->num_cu * 4 * kMegaSmallWaves)
-            return sc->stack <= 64 ? LaunchMegaT<64, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed)
-                                   : LaunchMegaT<192, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed);
+            return sc->stack == kStackSmall ? LaunchMegaT<kStackSmall, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed)
+                                   : LaunchMegaT<kStackLarge, 64, false, kMegaSmallWaves>(c, sc, film, P, s0, n_s, count, timed);
     }
     const bool in_l2 = TreeBytes(sc) <= kTreeL2;
     if (sc->stack == kStackSmall)
@@ -1189,7 +1189,7 @@ extern "C" int gy_render_light_tracing(gy_scene* s, const gy_camera_desc* cam, c
     if (sc->dev.n_sph > 0) return Fail(GY_ERR_UNSUPPORTED, "gy_render_light_tracing: scenes with spheres");
     const int64_t n = (int64_t)cam->width * cam->height * p->spp;
     if (n >= (1ll << 36)) return Fail(GY_ERR_UNSUPPORTED, "gy_render_light_tracing: more than 2^36 light paths");
-    if (sc->stats.max_depth + 1 > 64) return Fail(GY_ERR_UNSUPPORTED, "gy_render_light_tracing: BVH deeper than the traversal stack");
+    if (sc->stats.max_depth + 1 > kTreeLevels) return Fail(GY_ERR_UNSUPPORTED, "gy_render_light_tracing: BVH deeper than the traversal stack");
     PathParams P;
     rc = MakePathParams(c, sc, *cam, *p, &P);
     if (rc != GY_OK) return rc;
@@ -1347,8 +1347,8 @@ extern "C" int gy_count_visits(gy_scene* s, const gy_ray* rays, int64_t n, int64
     if (rc != GY_OK) return rc;
     if (n > 0) {
         const bool sph = sc->dev.n_sph > 0;
-        auto kern = sc->stack <= 64 ? (sph ? k_count_visits<64, true> : k_count_visits<64, false>)
-                                    : (sph ? k_count_visits<192, true> : k_count_visits<192, false>);
+        auto kern = sc->stack == kStackSmall ? (sph ? k_count_visits<kStackSmall, true> : k_count_visits<kStackSmall, false>)
+                                    : (sph ? k_count_visits<kStackLarge, true> : k_count_visits<kStackLarge, false>);
         hipLaunchKernelGGL(kern, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, sc->dev,
                            (const gy_ray*)c->rays.ptr, n, (unsigned long long*)c->ctr.ptr);
         rc = CheckLaunch(c, "k_count_visits");
@@ -1594,11 +1594,11 @@ extern "C" int gy_li_samples(gy_scene* s, const gy_camera_desc* cam, const gy_re
     if (rc == GY_OK) {
         const unsigned blocks = (unsigned)((n + 127) / 128);
         const bool env = sc->dev.env.w > 0;
-        auto kern = sc->stack <= 64 ? (env ? k_li_samples<64, true, false> : k_li_samples<64, false, false>)
-                                    : (env ? k_li_samples<192, true, false> : k_li_samples<192, false, false>);
+        auto kern = sc->stack == kStackSmall ? (env ? k_li_samples<kStackSmall, true, false> : k_li_samples<kStackSmall, false, false>)
+                                    : (env ? k_li_samples<kStackLarge, true, false> : k_li_samples<kStackLarge, false, false>);
         if (sc->dev.n_sph > 0)
-            kern = sc->stack <= 64 ? (env ? k_li_samples<64, true, true> : k_li_samples<64, false, true>)
-                                   : (env ? k_li_samples<192, true, true> : k_li_samples<192, false, true>);
+            kern = sc->stack == kStackSmall ? (env ? k_li_samples<kStackSmall, true, true> : k_li_samples<kStackSmall, false, true>)
+                                   : (env ? k_li_samples<kStackLarge, true, true> : k_li_samples<kStackLarge, false, true>);
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(128), 0, c->stream, sc->dev, P, n, (const int32_t*)dx, (const int32_t*)dy,
                            (const int32_t*)ds, (float*)dL, (float*)dr, (int32_t*)dd);
         rc = CheckLaunch(c, "k_li_samples");

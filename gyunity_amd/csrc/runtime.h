@@ -21,9 +21,12 @@ enum KernelCategory {
     kKernOther = 7
 };
 
-// Traversal stack capacities (entries per lane).  Binary trees are at most 63
-// levels deep, so the wide tree's three entries a level stay below kStackLarge.
+// Traversal stack capacities (entries per lane): at most three children a level
+// of the wide tree wait, and it has no more levels than the binary tree, which
+// scene creation limits to kTreeLevels.  No push checks the bound.
+constexpr int kTreeLevels = 64;
 constexpr int kStackSmall = 64, kStackLarge = 192;
+static_assert(3 * kTreeLevels <= kStackLarge, "the deepest tree's stack");
 
 struct DevBuf {
     void* ptr = nullptr;

@@ -590,7 +590,7 @@ extern "C" int gy_render_sppm(gy_scene* s, const gy_camera_desc* cam, const gy_s
     };
     int end_bit = 32;
     while ((1ll << (end_bit - 32)) < WH) ++end_bit;
-    const bool stack64 = sc->stack > 64;
+    const bool deep = sc->stack == kStackLarge;
     // Photon vertices: one list per iteration of a chunk of iterations traced
     // together (photons_per_launch photon paths per launch, about 4M by
     // default), grown and traced again when a list overflows; the chunk
@@ -630,11 +630,11 @@ extern "C" int gy_render_sppm(gy_scene* s, const gy_camera_desc* cam, const gy_s
                 }
                 n_iter = std::min(chunk, sp->iterations - iter0);
                 hipLaunchKernelGGL(k_u32_fill, dim3(1), dim3(256), 0, c->stream, vcount, 0u, (int64_t)n_iter);
-                if (stack64)
-                    hipLaunchKernelGGL(k_sppm_trace<192>, dim3(G1(photons * n_iter, 128)), dim3(128), 0, c->stream, sc->dev, P,
+                if (deep)
+                    hipLaunchKernelGGL(k_sppm_trace<kStackLarge>, dim3(G1(photons * n_iter, 128)), dim3(128), 0, c->stream, sc->dev, P,
                                        VtxDev{vtx, vcount, vcap}, iter0, n_iter, photons);
                 else
-                    hipLaunchKernelGGL(k_sppm_trace<64>, dim3(G1(photons * n_iter, 128)), dim3(128), 0, c->stream, sc->dev, P,
+                    hipLaunchKernelGGL(k_sppm_trace<kStackSmall>, dim3(G1(photons * n_iter, 128)), dim3(128), 0, c->stream, sc->dev, P,
                                        VtxDev{vtx, vcount, vcap}, iter0, n_iter, photons);
                 rc = CheckLaunch(c, "k_sppm_trace");
                 if (rc != GY_OK) break;
@@ -653,8 +653,8 @@ extern "C" int gy_render_sppm(gy_scene* s, const gy_camera_desc* cam, const gy_s
             if (rc != GY_OK) break;
         }
         // 1. eye pass
-        if (stack64) hipLaunchKernelGGL(k_sppm_eye<192>, dim3(G1(WH, 128)), dim3(128), 0, c->stream, sc->dev, P, D, iter);
-        else hipLaunchKernelGGL(k_sppm_eye<64>, dim3(G1(WH, 128)), dim3(128), 0, c->stream, sc->dev, P, D, iter);
+        if (deep) hipLaunchKernelGGL(k_sppm_eye<kStackLarge>, dim3(G1(WH, 128)), dim3(128), 0, c->stream, sc->dev, P, D, iter);
+        else hipLaunchKernelGGL(k_sppm_eye<kStackSmall>, dim3(G1(WH, 128)), dim3(128), 0, c->stream, sc->dev, P, D, iter);
         rc = CheckLaunch(c, "k_sppm_eye");
         if (rc != GY_OK) break;
         // 2. hash grid

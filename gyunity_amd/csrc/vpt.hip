@@ -1149,12 +1149,12 @@ int LaunchVpt(Ctx* c, Scene* sc, const PathParams& P, int s0, int n_s, bool eqa)
     const int64_t threads = (int64_t)tilesX * tilesY * 64 * n_s;
     const unsigned blocks = (unsigned)((threads + 127) / 128);
     const bool env = sc->dev.env.w > 0;
-    if (sc->stack <= 64) {
-        if (env) LaunchVptT<64, true>(c, sc, P, F, s0, n_s, eqa, blocks);
-        else LaunchVptT<64, false>(c, sc, P, F, s0, n_s, eqa, blocks);
+    if (sc->stack == kStackSmall) {
+        if (env) LaunchVptT<kStackSmall, true>(c, sc, P, F, s0, n_s, eqa, blocks);
+        else LaunchVptT<kStackSmall, false>(c, sc, P, F, s0, n_s, eqa, blocks);
     } else {
-        if (env) LaunchVptT<192, true>(c, sc, P, F, s0, n_s, eqa, blocks);
-        else LaunchVptT<192, false>(c, sc, P, F, s0, n_s, eqa, blocks);
+        if (env) LaunchVptT<kStackLarge, true>(c, sc, P, F, s0, n_s, eqa, blocks);
+        else LaunchVptT<kStackLarge, false>(c, sc, P, F, s0, n_s, eqa, blocks);
     }
     return CheckLaunch(c, "k_vpt");
 }
@@ -1438,12 +1438,12 @@ extern "C" int gy_vpt_li_samples(gy_scene* s, const gy_camera_desc* cam, const g
     if (rc == GY_OK) {
         const unsigned blocks = (unsigned)((n + 127) / 128);
         const bool env = sc->dev.env.w > 0, eqa = equiangular != 0;
-        auto pick = [&](auto k32, auto k64) { return sc->stack <= 64 ? k32 : k64; };
-        decltype(&k_vpt_li_samples<64, false, false>) kern;
-        if (env) kern = eqa ? pick(k_vpt_li_samples<64, true, true>, k_vpt_li_samples<192, true, true>)
-                            : pick(k_vpt_li_samples<64, true, false>, k_vpt_li_samples<192, true, false>);
-        else kern = eqa ? pick(k_vpt_li_samples<64, false, true>, k_vpt_li_samples<192, false, true>)
-                        : pick(k_vpt_li_samples<64, false, false>, k_vpt_li_samples<192, false, false>);
+        auto pick = [&](auto small, auto large) { return sc->stack == kStackSmall ? small : large; };
+        decltype(&k_vpt_li_samples<kStackSmall, false, false>) kern;
+        if (env) kern = eqa ? pick(k_vpt_li_samples<kStackSmall, true, true>, k_vpt_li_samples<kStackLarge, true, true>)
+                            : pick(k_vpt_li_samples<kStackSmall, true, false>, k_vpt_li_samples<kStackLarge, true, false>);
+        else kern = eqa ? pick(k_vpt_li_samples<kStackSmall, false, true>, k_vpt_li_samples<kStackLarge, false, true>)
+                        : pick(k_vpt_li_samples<kStackSmall, false, false>, k_vpt_li_samples<kStackLarge, false, false>);
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(128), 0, c->stream, sc->dev, MediaView(sc), P, n, (const int32_t*)dx,
                            (const int32_t*)dy, (const int32_t*)ds, (float*)dL, (float*)dr, (int32_t*)dd);
         rc = CheckLaunch(c, "k_vpt_li_samples");

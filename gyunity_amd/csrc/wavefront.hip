@@ -1219,7 +1219,7 @@ int WavefrontPass(Ctx* c, Scene* sc, const PathParams& P, const gy_render_params
         hipLaunchKernelGGL((k_wf_resolve<OneRender>), dim3(ResolveBlocks((uint32_t)cap)), dim3(256), 0, c->stream, Rd, W, (uint32_t)cap);
         return CheckLaunch(c, "k_wf_resolve");
     }
-    if (sc->stats.max_depth + 1 > 64) return Fail(GY_ERR_UNSUPPORTED, "BVH deeper than the traversal stack");
+    if (sc->stats.max_depth + 1 > kTreeLevels) return Fail(GY_ERR_UNSUPPORTED, "BVH deeper than the traversal stack");
     return WfBounceLoop<kStackLds>(c, Rd, W, p.max_depth, RefillOf(p.refill_threshold), p.ray_sort, blocks, (uint32_t)cap,
                                    sc->dev.env.w > 0, sc->mat_types, sc->film.counters);
 }
