@@ -721,7 +721,7 @@ int MakePathParamsFor(Ctx* c, Scene* sc, const gy_camera_desc& cam, const gy_ren
     P->rr_depth = p.rr_depth;
     if (p.sampler == GY_SAMPLER_SOBOL) {
         // dimensions a path may consume: 2 + depth * (6 + 3 + 1)
-        const int64_t dims = 2 + (int64_t)p.max_depth * 10;
+        const int64_t dims = kCameraDims + (int64_t)p.max_depth * kBounceDims;
         if (dims > sobol::kDims) return Fail(GY_ERR_UNSUPPORTED, "max_depth needs more Sobol dimensions than the table holds");
         const int bits = 2 * rt.log2res + (p.spp > 1 ? 32 - __builtin_clz((unsigned)(p.spp - 1)) : 0);
         if (bits > sobol::kCols) return Fail(GY_ERR_UNSUPPORTED, "sample index beyond 52 bits");
@@ -740,7 +740,8 @@ int MakePathParams(Ctx* c, Scene* sc, const gy_camera_desc& cam, const gy_render
 
 int ValidateRender(const gy_camera_desc* cam, const gy_render_params* p) {
     if (!cam || !p) return Fail(GY_ERR_INVALID, "render: null camera or params");
-    if (p->spp <= 0 || p->max_depth < 0 || p->max_depth > 100) return Fail(GY_ERR_INVALID, "render: spp > 0 and 0 <= max_depth <= 100");
+    if (p->spp <= 0 || p->max_depth < 0 || p->max_depth > kMaxPathDepth)
+        return Fail(GY_ERR_INVALID, "render: spp > 0 and 0 <= max_depth <= " + std::to_string(kMaxPathDepth));
     if ((int64_t)cam->width * cam->height > (1ll << 26)) return Fail(GY_ERR_UNSUPPORTED, "render: image larger than 2^26 pixels");
     if (p->sampler != GY_SAMPLER_SOBOL && p->sampler != GY_SAMPLER_HALTON) return Fail(GY_ERR_INVALID, "render: unknown sampler");
     if (p->ray_sort < GY_RAY_SORT_NONE || p->ray_sort > GY_RAY_SORT_OCTANT_LOCAL) return Fail(GY_ERR_INVALID, "render: unknown ray_sort");

@@ -28,6 +28,11 @@ constexpr int kTreeLevels = 64;
 constexpr int kStackSmall = 64, kStackLarge = 192;
 static_assert(3 * kTreeLevels <= kStackLarge, "the deepest tree's stack");
 
+// Path tracing and its kin: the longest path a caller may ask for, and the
+// sample dimensions that a camera ray and a bounce draw at most.
+constexpr int kMaxPathDepth = 100;
+constexpr int kCameraDims = 2, kBounceDims = 10;
+
 struct DevBuf {
     void* ptr = nullptr;
     size_t bytes = 0;

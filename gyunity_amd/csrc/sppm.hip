@@ -506,7 +506,7 @@ using namespace gy;
 extern "C" int gy_render_sppm(gy_scene* s, const gy_camera_desc* cam, const gy_sppm_params* sp, float* rgb, float* radius2,
                               float* photon_count) {
     if (!s || !cam || !sp || !rgb) return Fail(GY_ERR_INVALID, "gy_render_sppm: null argument");
-    if (sp->iterations <= 0 || sp->photons_per_iteration <= 0 || sp->max_depth <= 0 || sp->max_depth > 100 ||
+    if (sp->iterations <= 0 || sp->photons_per_iteration <= 0 || sp->max_depth <= 0 || sp->max_depth > kMaxPathDepth ||
         !(sp->initial_radius > 0.f) || !(sp->alpha > 0.f && sp->alpha <= 1.f))
         return Fail(GY_ERR_INVALID, "gy_render_sppm: iterations, photons, 0 < max_depth <= 100, radius > 0, 0 < alpha <= 1");
     if (sp->trace_glossy_ray) return Fail(GY_ERR_UNSUPPORTED, "gy_render_sppm: traceGlossyRay");

@@ -48,14 +48,16 @@ constexpr int C_WORDS = 64;
 // queues do not serialise on one L2 channel.
 constexpr int kCtrStride = 32;
 
-// Path state word (T.w): sample dimensions drawn (at most 2 + 100 * 10), depth
-// (at most 100), whether the last bounce was a delta one, and the film footprint
-// mask of the path's sample (film_mark).
+// Path state word (T.w): sample dimensions drawn, depth, whether the last bounce
+// was a delta one, and the film footprint mask of the path's sample (film_mark).
 constexpr uint32_t kStCursor = 0x7ffu;
 constexpr int kStDepth = 11;  // 7 bits
 constexpr uint32_t kStDepthMask = 0x7fu;
 constexpr uint32_t kStDelta = 1u << 18;
 constexpr int kStMask = 19;  // 9 bits
+static_assert(kCameraDims + kMaxPathDepth * kBounceDims <= (int)kStCursor, "cursor of the longest path");
+static_assert(kMaxPathDepth <= (int)kStDepthMask, "depth of the longest path");
+static_assert(kStCursor < (1u << kStDepth) && (kStDepthMask << kStDepth) < kStDelta && kStMask + 9 <= 32, "fields apart");
 __device__ inline uint32_t st_pack(uint32_t cursor, uint32_t depth, bool delta, uint32_t mask) {
     return cursor | (depth << kStDepth) | (delta ? kStDelta : 0u) | (mask << kStMask);
 }
