@@ -108,6 +108,8 @@ typedef struct {
     int32_t reserved[2];
 } gy_bvh_params;
 
+/* The builder's binary tree (gy_scene_bvh_download), from which the traversal
+ * tree is made. */
 typedef struct {
     int64_t n_nodes;
     int64_t n_leaves;
@@ -252,7 +254,10 @@ int gy_trace_any_device(gy_scene* scene, const gy_ray* rays_device, int64_t n, i
 /* Device time (ms) of the last trace kernel, measured with HIP events on the
  * stream it ran on. */
 double gy_last_kernel_ms(gy_context* ctx);
-/* Count BVH nodes and triangles the closest-hit traversal visits. */
+/* Nodes and triangles that the closest-hit traversal visits: nodes of the
+   four-wide traversal tree (64 bytes each, about half as many as the binary
+   nodes of gy_scene_stats and gy_scene_bvh_download), as the rays of a wave
+   walk it together (a lane that waits with a found leaf walks on). */
 int gy_count_visits(gy_scene* scene, const gy_ray* rays, int64_t n, int64_t* node_visits, int64_t* tri_visits);
 
 /* ---- rendering (Integrator::Render + Film::AddSample,
@@ -281,7 +286,8 @@ const char* gy_kernel_name(int index);
 int gy_li_samples(gy_scene* scene, const gy_camera_desc* cam, const gy_render_params* p, int32_t n,
                   const int32_t* x, const int32_t* y, const int32_t* s, float* L, float* raster, int32_t* dims);
 /* Algorithmic HBM traffic of a render: node/triangle visits of every traced ray
- * and shading points, counted by an instrumented copy of the kernels. */
+ * (nodes as gy_count_visits counts them) and shading points, counted by an
+ * instrumented copy of the megakernel. */
 int gy_count_traffic(gy_scene* scene, const gy_camera_desc* cam, const gy_render_params* p, gy_render_stats* out);
 
 /* ---- launch autotuner --------------------------------------------------------
