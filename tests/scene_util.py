@@ -469,3 +469,30 @@ def medium_cornell(res=64, spp=16, depth=8):
     cam.width = cam.height = res
     prm.spp, prm.max_depth, prm.rr_depth = spp, depth, depth
     return sa, cam, prm, media, tri
+
+
+def wide_levels(nodes):
+    """Levels of the four-wide tree made from the binary nodes of Scene.bvh(): a
+    node's two children, and while there is room the interior child of the
+    largest area gives way to its own two.  Its stack holds three entries a level."""
+    box = np.ascontiguousarray(nodes[:, :12]).view(np.float32).reshape(-1, 2, 6)
+    e = box[..., 3:] - box[..., :3]
+    area = e[..., 0] * e[..., 1] + e[..., 1] * e[..., 2] + e[..., 2] * e[..., 0]
+    ref, cnt = nodes[:, 12:14], nodes[:, 14:16]
+    level, levels = [0], 0
+    while level:
+        levels += 1
+        below = []
+        for node in level:
+            kids, at, opened = [], 0, node
+            while True:
+                new = [(area[opened, c], int(ref[opened, c]), int(cnt[opened, c])) for c in (0, 1) if ref[opened, c] != 0xffffffff]
+                kids[at:at + 1] = new
+                inner = [i for i, k in enumerate(kids) if k[2] == 0]
+                if len(kids) == 4 or not inner:
+                    break
+                at = max(inner, key=lambda i: kids[i][0])
+                opened = kids[at][1]
+            below += [k[1] for k in kids if k[2] == 0]
+        level = below
+    return levels
