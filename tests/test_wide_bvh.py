@@ -3,7 +3,9 @@ few nodes, trees deep enough to leave the LDS part of the stack, flat boxes,
 scenes away from the origin; rays along the axes, from far away, with
 directions of other lengths and with a finite range.  Boxes only decide which
 triangles are looked at, so the hit must be, bit for bit, the one that the FP32
-triangle test and its bounds gate give over all triangles."""
+triangle test and its bounds gate give over all triangles, as long as that test
+places no hit in front of its triangle's padded box (tiny nested triangles seen
+from far away: test_tiny_triangles_from_far_away)."""
 import numpy as np
 import pytest
 
@@ -142,6 +144,27 @@ def test_hits_are_the_brute_force_hits(gpu_ctx, kind, n, leaf):
     assert np.array_equal(hits["prim"], prim)
     assert np.array_equal(hits["t"], t) and np.array_equal(hits["b1"], b1) and np.array_equal(hits["b2"], b2)
     assert np.array_equal(any_hit, occluded)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("leaf", [1, 4])
+@pytest.mark.parametrize("far", [4.0, 40.0, 400.0])
+def test_tiny_triangles_from_far_away(gpu_ctx, far, leaf):
+    # The triangle test's FP32 distance can be off by more than its box is
+    # padded, so the traversal can find a triangle close behind first and then
+    # pass the box by.  2 to 9 of about 4500 hits; the bound is four times
+    # the largest.  What is found is a hit, behind the nearest, and whether there
+    # is one does not depend on it.
+    rng = np.random.default_rng(150 + leaf)
+    tri = soup("chain", 150, rng)
+    rays = rays_for(tri, 8000, rng, far)
+    t, prim, _, _, occluded = (np.concatenate(p) for p in zip(*(brute_force(tri, r) for r in np.array_split(rays, 20))))
+    with g.Scene(gpu_ctx, scene(tri), max_leaf_size=leaf) as sc:
+        hits, any_hit = sc.trace_closest(rays), sc.trace_any(rays)
+    assert np.array_equal(any_hit, occluded) and np.array_equal(hits["prim"] >= 0, prim >= 0)
+    other = hits["prim"] != prim
+    assert other.sum() <= 36 and (hits["t"][other] >= t[other]).all()
+    assert np.array_equal(hits["t"][~other], t[~other])
 
 
 @pytest.mark.gpu
