@@ -36,14 +36,15 @@ def kernel_bytes(name, st, paths):
         # all traversals, material records, the radiance record of each sample
         return 64.0 * st.node_visits + 48.0 * st.tri_visits + 16.0 * st.shade_points + 16.0 * paths
     if name == "wf_trace_closest":
-        # + ray (32 B) read, hit (16 B) written, queue entry read and pushed
-        return 64.0 * nv[0] + 48.0 * tv[0] + 56.0 * primary
+        # + queue entry (4 B) and ray (24 B) read, hit (12 B) and its material type (1 B) written
+        return 64.0 * nv[0] + 48.0 * tv[0] + 41.0 * primary
     if name == "wf_trace_shadow_mis":
-        # shadow rays, then MIS rays, in one launch
-        return 64.0 * (nv[1] + nv[2]) + 48.0 * (tv[1] + tv[2]) + 36.0 * (st.shadow_rays + st.mis_rays)
+        # shadow rays (28 B), then MIS rays (24 B), in one launch: + queue entry (4 B), a shadow ray's flag (4 B)
+        return 64.0 * (nv[1] + nv[2]) + 48.0 * (tv[1] + tv[2]) + 36.0 * st.shadow_rays + 28.0 * st.mis_rays
     if name == "wf_shade":
-        # shading record 128 B, material 128 B, path state ~200 B per shading point
-        return 456.0 * st.shade_points
+        # shading record 128 B, material 128 B; of the path state 64 B read and 84 B written
+        # by a point that sends a shadow ray and goes on
+        return 404.0 * st.shade_points
     return float("nan")
 
 
