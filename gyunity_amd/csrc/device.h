@@ -685,7 +685,8 @@ struct SpillPrivate {
 // to 1e24.
 GY_D int ray_exponent(V3 d) {
     const float m = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
-    return (m >= 1e-24f && m <= kDirMin) || (m >= kDirMax && m <= 1e24f) ? -ilogbf(m) : 0;
+    if (__builtin_expect(m > kDirMin && m < kDirMax, 1)) return 0;
+    return m >= 1e-24f && m <= 1e24f ? 1 - __builtin_amdgcn_frexp_expf(m) : 0;
 }
 // QUERY: the ray is a caller's, whose direction may have any length.
 template <bool ANY, int STACK, bool COUNT = false, bool SPH = false, bool QUERY = false>
