@@ -879,10 +879,10 @@ def main():
         # HBM bytes the counters measured per launch over the live launch time
         "measured_hbm_gbs": round(traffic / (avg_launch_ms / 1e3) / 1e9, 2) if traffic else None,
         "measured_hbm_frac": round(traffic / (avg_launch_ms / 1e3) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
-        "limiter": "VALU with divergent lanes, 0.47 busy per instruction (profiles/counters_icosphere-L8-1024-64spp.txt), "
-                   "and the L1's address rate: the upper BVH levels are re-read from L2 and the Infinity Cache, so "
-                   "counter-measured HBM bytes are about half the algorithmic bytes, and the algorithmic rate (frac) can "
-                   "pass HBM's peak",
+        "limiter": "VALU with divergent lanes, 96% busy at 0.47 lanes per instruction, the L1's address unit 72% busy "
+                   "(profiles/counters_icosphere-L8-1024-64spp.txt): the upper BVH levels are re-read from L2 and the "
+                   "Infinity Cache, so counter-measured HBM bytes are about half the algorithmic bytes, and the "
+                   "algorithmic rate (frac) can pass HBM's peak",
         "algorithmic_bytes_per_launch": bytes_per_launch,
         "avg_launch_ms": round(avg_launch_ms, 4),
         "launches_per_step": launches_per_step,

@@ -541,12 +541,13 @@ GY_D void trav_swap(float& ka, uint32_t& ea, float& kb, uint32_t& eb) {
 // leaves together, and a second leaf met on the way, while the few still
 // searching wait and resume in the next round.
 //
-// What bounds it: the L1's address rate.  A wave's lanes visit different nodes,
-// and the L1 takes about one lane's 16 bytes a cycle, so loads per ray count
-// first and VALU instructions second.  A node therefore holds four children in
-// 64 bytes (four loads; two-wide FP32 nodes took four for two children, four
-// wide ones in FP32 seven), and one pass of the loop with its stack and leaf
-// bookkeeping serves four boxes.  A byte plane costs half a byte permute, which
+// What bounds it: VALU issue with half the lanes busy (96% of the time in the
+// closest-hit trace), and close behind it the L1's address unit (72%).  A wave's
+// lanes visit different nodes, and the L1 takes about one lane's 16 bytes a
+// cycle: with 128-byte nodes it was 95% busy and came first.  A node therefore
+// holds four children in 64 bytes (four loads; two-wide FP32 nodes took four for
+// two children, four wide ones in FP32 seven), and one pass of the loop with its
+// stack and leaf bookkeeping serves four boxes.  A byte plane costs half a byte permute, which
 // also picks near or far, and one mixed-precision FMA.
 // The slab test only decides which triangles are looked at, and ref_triangle in
 // FP32 which are hit.  Boxes are padded (4e-6 (1 + extent)) and rounded outward,
