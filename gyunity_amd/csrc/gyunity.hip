@@ -790,7 +790,7 @@ int LaunchMegaBlock(Ctx* c, Scene* sc, const FilmState& film, const PathParams& 
 // instantiation when the pass has no more waves than that keeps resident; such
 // a launch is a chain of latencies, spilled registers are on it, and its waves
 // spread over twice the CUs.  64 to 3072 waves of depth 6, against five waves a
-// SIMD and 128 threads: Cornell room 0.32 -> 0.30 ms at 256 waves, 0.39 -> 0.32
+// SIMD and 128 threads: Cornell room 0.35 -> 0.30 ms at 256 waves, 0.39 -> 0.32
 // at 1024, 0.58 -> 0.42 at 3072; 1.31M triangles 1.01 -> 0.92, 1.07 -> 0.99,
 // 1.31 -> 1.15; 5,132 and 82k triangles between those.
 //
