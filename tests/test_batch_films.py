@@ -13,7 +13,7 @@ import gyunity_amd as g
 def test_films_of_ragged_entries(gpu_ctx, sizes, use_graph):
     sa, _, _ = g.generate_scene(g.GY_SCENE_CORNELL, 0, 64)
     with g.Scene(gpu_ctx, sa) as sc, g.Batch(gpu_ctx, use_graph=use_graph) as b:
-        views = [(g.camera((0.0, 1.0, 3.4), (0.0, 1.0, 0.0), (0, 1, 0), 45.0, w, h),
+        views = [(g.camera((0.5, 0.5, 2.35), (0.5, 0.5, 0.0), (0, 1, 0), 40.0, w, h),
                   g.render_params(5 + 27 * i, 3, mode=g.GY_RENDER_WAVEFRONT, samples_per_pass=5 + 27 * i))
                  for i, (w, h) in enumerate(sizes)]
         refs = [sc.render(cam, prm) for cam, prm in views]
@@ -24,4 +24,6 @@ def test_films_of_ragged_entries(gpu_ctx, sizes, use_graph):
                 got = b.film(e)
                 assert np.array_equal(got[1], weight) and np.array_equal(got[0], color)
             sc.render(*views[0])
-        assert all(w.sum() > 0 for _, w in refs)
+        assert all(c.sum() > 0 for c, _ in refs)
+        # samples on pixel borders count in more than one pixel
+        assert len(sizes) == 1 or any((w > 5 + 27 * i).any() for i, (_, w) in enumerate(refs))

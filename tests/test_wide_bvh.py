@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import gyunity_amd as g
-from gyunity_amd._lib import FAULT_SYNC, GY_ERR_INJECTED
+from gyunity_amd._lib import FAULT_LAUNCH, FAULT_SYNC, GY_ERR_INJECTED
 from tests.scene_util import wide_levels
 
 def soup(kind, n, rng):
@@ -260,14 +260,16 @@ def test_both_builders_trees_give_the_same_hits(gpu_ctx, kind, n):
 
 
 @pytest.mark.gpu
-def test_a_tree_whose_copy_failed_makes_no_scene(gpu_ctx):
-    # the device's tree is copied out of the build's workspace last; traversal
-    # follows its indices without bounds checks
-    sa, _, _ = g.generate_scene(g.GY_SCENE_ICOSPHERE_GGX, 1, 6)
-    gpu_ctx.inject_fault(FAULT_SYNC)
+@pytest.mark.parametrize("level,builder,fault", [(6, 0, FAULT_SYNC), (6, 1, FAULT_SYNC), (5, 1, FAULT_LAUNCH), (6, 1, FAULT_LAUNCH)])
+def test_a_tree_that_failed_on_the_device_makes_no_scene(gpu_ctx, level, builder, fault):
+    # a large tree is copied out of the build's workspace last (the wait for it
+    # fails); the first launch of the host's builds is the collapse.  Traversal
+    # follows the tree's indices without bounds checks
+    sa, _, _ = g.generate_scene(g.GY_SCENE_ICOSPHERE_GGX, 1, level)
+    gpu_ctx.inject_fault(fault)
     with pytest.raises(g.GyError) as e:
-        g.Scene(gpu_ctx, sa)
+        g.Scene(gpu_ctx, sa, builder=builder)
     assert e.value.code == GY_ERR_INJECTED
     rays = rays_for(sa.pos.reshape(-1, 3, 3), 1000, np.random.default_rng(0))
-    with g.Scene(gpu_ctx, sa) as sc:
+    with g.Scene(gpu_ctx, sa, builder=builder) as sc:
         assert (sc.trace_closest(rays)["prim"] >= 0).mean() > 0.2
